@@ -356,9 +356,10 @@ __global__ void count_tokens_kernel(const int32_t* __restrict__ token_map, int S
 
 // Exclusive scan of n ints in one workgroup of 1024 threads (contiguous chunk
 // per thread). Writes out[0..n] (out[n] = total) and a copy into cursor[0..n).
+// cursor may be `in` itself, so each count is read before its slot is written
+// and neither pointer is restrict.
 __global__ __launch_bounds__(kScanThreads) void scan_generic_kernel(
-    const int32_t* __restrict__ in, int n, int32_t* __restrict__ out,
-    int32_t* __restrict__ cursor) {
+    const int32_t* in, int n, int32_t* __restrict__ out, int32_t* cursor) {
   __shared__ int s_wave[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int per = (n + kScanThreads - 1) / kScanThreads;
@@ -372,9 +373,10 @@ __global__ __launch_bounds__(kScanThreads) void scan_generic_kernel(
   for (int w = 0; w < wave; ++w) wpre += s_wave[w];
   int run = wpre + inc - local;
   for (int i = i0; i < i1; ++i) {
+    const int c = in[i];
     out[i] = run;
     if (cursor != nullptr) cursor[i] = run;
-    run += in[i];
+    run += c;
   }
   if (tid == kScanThreads - 1) out[n] = run;
 }

@@ -141,6 +141,16 @@ def test_combine_random_token_map(dsk, T):
     _combine_case(dsk, y, tm, dw, T)
 
 
+@pytest.mark.parametrize("T", [1023, 1024, 1025, 2005, 3001, 5000])
+def test_combine_more_tokens_than_scan_threads(dsk, T):
+    """From 1024 tokens up a thread of the prefix sum owns several counts, which it
+    overwrites with the cursors as it goes."""
+    g = torch.Generator().manual_seed(20 + T)
+    y = torch.randn(T * 2, 64, generator=g).to(torch.bfloat16)
+    tm = torch.randint(0, T, (T * 2,), generator=g, dtype=torch.int32)
+    _combine_case(dsk, y, tm, torch.rand(T * 2, generator=g), T)
+
+
 def test_combine_single_and_multi_slot(dsk):
     g = torch.Generator().manual_seed(0)
     T = 64
