@@ -63,6 +63,30 @@ __device__ __forceinline__ void rope_pair(float x0, float x1, float c_lo, float 
   hi = x1 * c_hi + x0 * s_hi;
 }
 
+// Pieces g and 4 + g (elements 8g..8g+7 and 32+8g..32+8g+7) of the rotated
+// 64-wide RoPE vector, from the raw elements 16g..16g+15 (x, two 16-byte
+// pieces) and the angles cos/sin[8g..8g+7] and [32+8g..32+8g+7] of its position.
+__device__ __forceinline__ void rope_pieces(const u32x4_t (&x)[2], u32x4_t clo, u32x4_t chi,
+                                            u32x4_t slo, u32x4_t shi, u32x4_t& lo_piece,
+                                            u32x4_t& hi_piece) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {  // output pair (2e, 2e+1) of each piece
+    float lo[2], hi[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int j = 2 * e + u;                 // element 8g + j: raw pair j
+      const uint32_t xr = x[j >> 2][j & 3];    // (x[2k], x[2k+1]) with k = 8g + j
+      const float cl = u ? bf16hi(clo[e]) : bf16lo(clo[e]);
+      const float ch = u ? bf16hi(chi[e]) : bf16lo(chi[e]);
+      const float sl = u ? bf16hi(slo[e]) : bf16lo(slo[e]);
+      const float sh = u ? bf16hi(shi[e]) : bf16lo(shi[e]);
+      rope_pair(bf16lo(xr), bf16hi(xr), cl, ch, sl, sh, lo[u], hi[u]);
+    }
+    lo_piece[e] = pack_bf16x2(lo[0], lo[1]);
+    hi_piece[e] = pack_bf16x2(hi[0], hi[1]);
+  }
+}
+
 // ------------------------------------------------- memory-counter helpers --
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding:
 // vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]).

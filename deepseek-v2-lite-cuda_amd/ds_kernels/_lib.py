@@ -57,6 +57,9 @@ SIGNATURES = {
     "dsk_mla_decode_attention": (_I, [_P, _I64, _I64, _P, _I64, _I64, _P, _P, _P, _I, _I64,
                                       _I64, _P, _P, _F, _F, _I, _I, _I, _P, _I64, _I64, _P, _SZ,
                                       _P]),
+    "dsk_mla_prefill_attention": (_I, [_P, _I64, _P, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _F,
+                                       _I, _P, _I, _I64, _I64, _I64, _P, _I64, _I, _I, _I, _I,
+                                       _P]),
     "dsk_rms_norm": (_I, [_P, _I64, _P, _P, _I64, _I, _I, _F, _P]),
     "dsk_rms_norm_f32": (_I, [_P, _I64, _P, _P, _I64, _I, _I, _F, _P]),
     "dsk_rope": (_I, [_P, _I64, _I64, _I64, _P, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),

@@ -7,10 +7,10 @@ layout) for q_proj, kv_a_proj_with_mqa and o_proj, `rms_norm` straight on the
 512-wide latent slice of the 576-wide kv_a output (row-strided, no copy),
 `kv_upproj`, `rope` on strided q_pe / k_pe views with the position tables
 broadcast over the batch (no materialised copies), and the fused MoE layer
-(`moe_layer_forward`). In the causal attention core the two batched products
-stay torch (the attention core is outside the kernel scope); the scale, causal mask, fp32 softmax and
-bf16 rounding between them are one pass of `attn_softmax_`, at the reference's
-precision.
+(`moe_layer_forward`). The attention core is one kernel, `mla_prefill_attention`,
+on the projection rows; head dims other than 128 + 64 / 128 take torch's batched
+products with the scale, causal mask, fp32 softmax and bf16 rounding between
+them in one pass of `attn_softmax_`.
 """
 from __future__ import annotations
 
@@ -196,27 +196,29 @@ def mla_forward(x: torch.Tensor, W: MLAWeights, cos: torch.Tensor, sin: torch.Te
                 eps: float = 1e-6, attention_mask: Optional[torch.Tensor] = None,
                 position_ids: Optional[torch.Tensor] = None) -> torch.Tensor:
     """DeepSeekMLA.forward (mla.py:295-393): projections on this package's
-    kernels, o_proj on the MFMA GEMM, and the attention core at the
-    reference's precision (mla.py:366-384): bf16 Q.K^T and .V in torch
-    (right-hand operands contiguous), the scale, mask, fp32 softmax and bf16
-    rounding in one pass of attn_softmax_.
+    kernels, o_proj on the MFMA GEMM, and the attention core (mla.py:354-384) in
+    one kernel on the projection rows, with the scores in fp32 and the
+    probabilities rounded to bf16 for the product with V, as in the reference.
     x: bf16 [b, s, H] -> bf16 [b, s, H], any s >= 1. cos/sin: the YaRN tables
     for positions 0.. (at least s rows). attention_mask: additive [b, 1, s, s]
     (bf16 or fp32, -inf where masked; anything broadcastable to it) used instead
     of the causal mask, as in the reference; position_ids: [b, s] rows of the
-    tables for each token (default 0..s-1). With s % 8 != 0 the key dimension of
-    K^T, the scores and V is padded to a multiple of 8 with zeros."""
+    tables for each token (default 0..s-1)."""
     b, s, H = x.shape
-    h, nope, r = W.n_heads, W.nope, W.rope_dim
+    h, r = W.n_heads, W.rope_dim
     cs, sn = rope_tables_for(cos, sin, s, position_ids)
-    sp = (s + 7) // 8 * 8
-    if (nope, r, W.v_dim) == (128, 64, 128):
-        # Q, K^T and V packed head-major in one pass from the projection rows
-        # (RoPE of q_pe and k_pe included); other head dims assemble them by copies
+    if (W.nope, r, W.v_dim) == (128, 64, 128):
         qr, kv, kva, _ = _projection_rows(x, W, eps, with_latent=False)
-        q, kT, v = ops.mla_attn_pack(qr, kv, kva[..., W.kv_lora:], cs, sn, heads=h, pad=True)
-    else:
-        q, kT, v = _assemble_attention_operands(x, W, cs, sn, eps, sp)
+        cs, sn = cs.contiguous(), sn.contiguous()
+        ct, st = ((t if t.dim() == 3 else t[None])[:, None].expand(b, 1, s, r) for t in (cs, sn))
+        k_rot = ops.rope_single(kva[:, None, :, W.kv_lora:], ct, st)[:, 0]
+        o = ops.mla_prefill_attention(qr, kv, k_rot, cs, sn, W.softmax_scale, heads=h,
+                                      causal=attention_mask is None, mask=attention_mask)
+        return ops.linear(o, W.o)
+    # other head dims: K^T, the scores and V with the key dimension padded to a
+    # multiple of 8 with zeros
+    sp = (s + 7) // 8 * 8
+    q, kT, v = _assemble_attention_operands(x, W, cs, sn, eps, sp)
     scores = torch.matmul(q, kT)                                       # bf16 [b,h,s,sp]
     p = ops.attn_softmax_(scores, W.softmax_scale, causal=attention_mask is None, kv_len=s,
                           mask=attention_mask)
@@ -227,7 +229,7 @@ def mla_forward(x: torch.Tensor, W: MLAWeights, cos: torch.Tensor, sin: torch.Te
 
 def _assemble_attention_operands(x, W: MLAWeights, cs, sn, eps, sp):
     """Q [b,h,s,nope+r], K^T [b,h,nope+r,sp] and V [b,h,sp,v] by copies, for head
-    dims the pack kernel does not take; K^T columns and V rows past s are zero."""
+    dims the fused kernel does not take; K^T columns and V rows past s are zero."""
     b, s, _ = x.shape
     h, nope, r = W.n_heads, W.nope, W.rope_dim
     q_nope, q_rot, k_nope, v, k_rot, _ = mla_projections(x, W, cs, sn, eps, with_latent=False)

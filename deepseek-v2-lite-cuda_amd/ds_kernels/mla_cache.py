@@ -214,16 +214,23 @@ ROWS_MAX_TOKENS = 4
 def _attend_up_projected(q: torch.Tensor, cache: LatentKVCache, W: MLAWeights, cos: torch.Tensor,
                          sin: torch.Tensor, eps: float) -> torch.Tensor:
     """The attention of mla.py:338-384 for the last n of the L cached positions:
-    RMSNorm of the cached latents, kv_b, RoPE of the cached keys and the new
-    queries, bf16 Q.K^T, attn_softmax_ (scale, causal mask offset by L - n, fp32
-    softmax), .V. q: [b, n, h, nope + rope] view of the q projection. Returns
-    bf16 [b, n, h * v_dim]."""
+    RMSNorm of the cached latents, kv_b, RoPE of the keys not rotated yet, and the
+    fused attention over them (causal, offset by L - n). q: [b, n, h, nope + rope]
+    view of the q projection. Returns bf16 [b, n, h * v_dim]."""
     b, n, h, _ = q.shape
     nope, r, vd = W.nope, W.rope_dim, W.v_dim
     L = cache.current_len
     lat, pe = cache.get(L)
-    kv = ops.kv_upproj(ops.rms_norm(lat, W.kva_norm, eps), W.kvb).view(b, L, h, nope + vd)
-    kv = kv.transpose(1, 2)                                       # [b, h, L, 256] view
+    kv = ops.kv_upproj(ops.rms_norm(lat, W.kva_norm, eps), W.kvb)       # [b, L, h * 256]
+    if (nope, r, vd) == (128, 64, 128):
+        l0 = cache.rope_len
+        if l0 < L:
+            ck, sk = (t[l0:L][None, None].expand(b, 1, L - l0, r) for t in (cos, sin))
+            cache.k_rope[:, l0:L].copy_(ops.rope_single(pe[:, None, l0:L], ck, sk)[:, 0])
+        cache._rope_len = L
+        return ops.mla_prefill_attention(q.reshape(b, n, h * (nope + r)), kv, cache.k_rope[:, :L],
+                                         cos[:L], sin[:L], W.softmax_scale, heads=h)
+    kv = kv.view(b, L, h, nope + vd).transpose(1, 2)              # [b, h, L, 256] view
     cq = cos[L - n:L][None, None].expand(b, 1, n, r)
     sq = sin[L - n:L][None, None].expand(b, 1, n, r)
     ck = cos[:L][None, None].expand(b, 1, L, r)

@@ -544,6 +544,21 @@ def _rope_strides(t: torch.Tensor, name: str):
     return sb, (sh if h > 1 else 0), ss
 
 
+def _expand_mask(op: str, mask: torch.Tensor, device, b: int, h: int, q_len: int,
+                 kv_len: int) -> torch.Tensor:
+    """An additive mask as a [b, h, q_len, kv_len] view with unit key stride."""
+    _req(mask.is_cuda and mask.device == device, f"{op}: mask must be on the scores' device.")
+    _req(mask.dtype in (torch.bfloat16, torch.float32), f"{op}: mask must be bf16 or fp32.")
+    _req(mask.dim() <= 4, f"{op}: mask must have at most 4 dims.")
+    m = mask.reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
+    try:
+        m = m.expand(b, h, q_len, kv_len)
+    except RuntimeError:
+        raise RuntimeError(f"{op}: mask {tuple(mask.shape)} does not broadcast to "
+                           f"[{b}, {h}, {q_len}, {kv_len}].") from None
+    return m if m.stride(-1) == 1 else m.contiguous()
+
+
 def attn_softmax_(scores: torch.Tensor, scale: float, causal: bool = True,
                   kv_len: int = None, mask: torch.Tensor = None) -> torch.Tensor:
     """In place over bf16 scores [..., q_len, L] (last dim contiguous, rows
@@ -577,18 +592,8 @@ def attn_softmax_(scores: torch.Tensor, scale: float, causal: bool = True,
                                        1 if causal else 0, st), op)
         return scores
     _req(scores.dim() == 4, f"{op}: a mask needs 4-D scores [b, h, q_len, L].")
-    _req(mask.is_cuda and mask.device == scores.device, f"{op}: mask must be on the scores' device.")
-    _req(mask.dtype in (torch.bfloat16, torch.float32), f"{op}: mask must be bf16 or fp32.")
     b, h = scores.shape[0], scores.shape[1]
-    _req(mask.dim() <= 4, f"{op}: mask must have at most 4 dims.")
-    m = mask.reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
-    try:
-        m = m.expand(b, h, q_len, kv_len)
-    except RuntimeError:
-        raise RuntimeError(f"{op}: mask {tuple(mask.shape)} does not broadcast to "
-                           f"[{b}, {h}, {q_len}, {kv_len}].") from None
-    if m.stride(-1) != 1:
-        m = m.contiguous()
+    m = _expand_mask(op, mask, scores.device, b, h, q_len, kv_len)
     with torch.cuda.device(scores.device):
         check(lib.dsk_attn_softmax_masked(
             flat.data_ptr(), L, rows, kv_len, q_len, h, float(scale), 1 if causal else 0,
@@ -642,6 +647,56 @@ def mla_attn_pack(q: torch.Tensor, kv: torch.Tensor, k_pe: torch.Tensor, cos: to
                                        k_t.data_ptr(), v.data_ptr(), b, s, sp, heads, 128, 64,
                                        128, stream_handle(dev)), op)
     return q_out, k_t, v
+
+
+def mla_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Tensor,
+                          cos: torch.Tensor, sin: torch.Tensor, scale: float, heads: int = 16,
+                          causal: bool = True, mask: torch.Tensor = None) -> torch.Tensor:
+    """The attention of DeepSeekMLA.forward (mla.py:354-384) for the last n of L
+    positions, fused: softmax(scale * (q_nope|rope(q_pe)) . (k_nope|k_rope) + mask) v
+    per head, the scores in fp32 registers throughout.
+    q: bf16 [b, n, h*192] (q_proj rows, each head nope then raw RoPE part), kv: bf16
+    [b, L, h*256] (kv_b_proj rows, each head k_nope then v), k_rope: bf16 [b, L, 64]
+    rotated shared keys; q and kv may have strided rows evenly spaced over batch and
+    sequence, k_rope any row and batch stride. cos/sin: tables by position ([>= L, 64]
+    or [b, >= L, 64]), used as bf16; query i is at position L - n + i. causal: query i
+    sees keys j <= i + L - n. mask: additive (bf16 or fp32), broadcastable to
+    [b, h, n, L]. Returns bf16 [b, n, h*128]."""
+    op = "mla_prefill_attention"
+    for t, nm in ((q, "q"), (kv, "kv"), (k_rope, "k_rope")):
+        _req(isinstance(t, torch.Tensor) and t.is_cuda, f"{op}: {nm} must be a CUDA tensor.")
+        _dtype(t, torch.bfloat16, nm, op)
+        _req(t.dim() == 3 and t.stride(2) == 1, f"{op}: {nm} must be 3-D with a contiguous last dim.")
+    b, n, nq = q.shape
+    L = kv.shape[1]
+    _req(nq == heads * 192 and kv.shape == (b, L, heads * 256) and k_rope.shape == (b, L, 64),
+         f"{op}: expected q [b, n, {heads}*192], kv [b, L, {heads}*256], k_rope [b, L, 64].")
+    _req(n <= L, f"{op}: {n} queries but only {L} keys.")
+    for t, nm in ((q, "q"), (kv, "kv")):
+        _req(b <= 1 or t.stride(0) == t.shape[1] * t.stride(1),
+             f"{op}: {nm} rows must be evenly spaced over batch and sequence.")
+    dev = q.device
+    for t, nm in ((cos, "cos"), (sin, "sin")):
+        _req(isinstance(t, torch.Tensor) and t.is_cuda, f"{op}: {nm} must be a CUDA tensor.")
+    cb, sb = cos.to(torch.bfloat16).contiguous(), sin.to(torch.bfloat16).contiguous()
+    _req(sb.shape == cb.shape and cb.dim() in (2, 3) and cb.shape[-2] >= L and cb.shape[-1] == 64
+         and (cb.dim() == 2 or cb.shape[0] == b),
+         f"{op}: cos/sin must be [>= {L}, 64] or [b, >= {L}, 64].")
+    m = _expand_mask(op, mask, dev, b, heads, n, L) if mask is not None else None
+    out = torch.empty((b, n, heads * 128), dtype=torch.bfloat16, device=dev)
+    if out.numel() == 0:
+        return out
+    with torch.cuda.device(dev):
+        check(lib.dsk_mla_prefill_attention(
+            q.data_ptr(), q.stride(1), kv.data_ptr(), kv.stride(1), k_rope.data_ptr(),
+            k_rope.stride(1), k_rope.stride(0), cb.data_ptr(), sb.data_ptr(), cb.stride(-2),
+            cb.stride(0) if cb.dim() == 3 else 0, float(scale), 1 if causal else 0,
+            m.data_ptr() if m is not None else None,
+            1 if m is not None and m.dtype == torch.float32 else 0,
+            m.stride(0) if m is not None else 0, m.stride(1) if m is not None else 0,
+            m.stride(2) if m is not None else 0, out.data_ptr(), heads * 128, b, n, L, heads,
+            stream_handle(dev)), op)
+    return out
 
 
 def _rows_overlap(a: torch.Tensor, wa: int, b: torch.Tensor, wb: int) -> bool:

@@ -218,6 +218,31 @@ int dsk_linear_rowscale(const dsk_bf16* x, int64_t ld_x, const dsk_bf16* w_tiled
                         const float* row_sumsq, int64_t ld_rowsq, int n_parts,
                         int n_cols, float eps, void* stream);
 
+/* ------------------------------------------------------ prefill attention --
+ * The attention of DeepSeekMLA.forward (mla.py:354-384) for the last q_len of
+ * kv_len positions, fused: scores and softmax in fp32 registers, probabilities
+ * rounded to bf16 for the product with V.
+ *   q: bf16 rows b * q_len + i at ld_q, per head 128 nope | 64 raw RoPE values;
+ *   kv: bf16 rows b * kv_len + j at ld_kv, per head 128 k_nope | 128 v;
+ *   k_rope: bf16 rotated shared keys, row (b, j) at b * kr_batch_stride + j * ld_kr;
+ *   cos/sin: bf16 tables by position (query i is at kv_len - q_len + i), row p of
+ *     batch entry b at b * cs_batch_stride + p * ld_cs (stride 0: shared);
+ *   causal: query i sees keys j <= i + kv_len - q_len;
+ *   mask: NULL, or an additive mask (DSK_DTYPE_BF16 / DSK_DTYPE_F32) with element
+ *     strides by batch entry, head and query and key stride 1; a query with every
+ *     key at -inf comes out NaN, as softmax does;
+ *   out: bf16 rows b * q_len + i at ld_out, per head 128 values.
+ * scale > 0; rows 16-byte aligned. */
+int dsk_mla_prefill_attention(const dsk_bf16* q, int64_t ld_q, const dsk_bf16* kv,
+                              int64_t ld_kv, const dsk_bf16* k_rope, int64_t ld_kr,
+                              int64_t kr_batch_stride, const dsk_bf16* cos_t,
+                              const dsk_bf16* sin_t, int64_t ld_cs,
+                              int64_t cs_batch_stride, float scale, int causal,
+                              const void* mask, int mask_dtype, int64_t mask_sb,
+                              int64_t mask_sh, int64_t mask_sq, dsk_bf16* out,
+                              int64_t ld_out, int batch, int q_len, int kv_len, int heads,
+                              void* stream);
+
 /* --------------------------------------------------------------- rms_norm --
  * y = w * x * rsqrt(mean(x^2) + eps), fp32 math, one rounding of the output.
  * bf16 in/out with fp32 weight: replaces launch_rms_norm
