@@ -25,8 +25,9 @@ struct GemmArgs {
   int offsets_sorted;      // offsets never decrease (the fused layer's own): the small-
                            // group grid then launches min(G, M) group ordinals, else G
   int chunk_m_tiles;       // large-group kernels: M tiles of a typical group, so that
-                           // tiles are dealt to the XCDs a group at a time (0: chunks
-                           // of kTileChunk tiles; gemm_sched.hpp sched_chunk)
+                           // tiles are dealt to the XCDs a group at a time (0: chunks of
+                           // up to kTileChunk tiles; gemm_sched.hpp)
+  int chunk;               // tiles per chunk of the deal (set by the launchers)
   int64_t a_group_stride;  // skinny kernel: elements between the A bases of consecutive
   int64_t c_group_stride;  // groups, and of the C bases (0: one base, rows by offsets)
   int b_tiled;             // B stored as MFMA fragments (see the fragment-tiled layout in
@@ -34,8 +35,8 @@ struct GemmArgs {
   uint16_t* C2;            // skinny kernel, optional: output columns n >= n_split go to
   int64_t ldc2;            // C2[m * ldc2 + n - n_split] instead of C (n_split % 64 == 0)
   int n_split;
-  // Row statistics in the epilogue of the one-wave-per-SIMD kernel (G = 1, no
-  // SwiGLU, no gather), optional:
+  // Row statistics in the epilogue of the medium-problem kernel (G = 1, no SwiGLU,
+  // no gather), optional:
   //   rowsq_out[(n0 - rowsq_c0) / 256 * ld_rowsq + m] = sum over the 256 output
   //   columns n0.. of tile n0 (inside [rowsq_c0, rowsq_c1)) of bf16(C[m, n])^2;
   //   rowscale_ss != NULL: C[m, :] *= rsqrt(sum_p rowscale_ss[p * ld_rowscale + m]
@@ -74,6 +75,11 @@ constexpr int kRouteInGemmTokens = 1;
 constexpr int kRouteInGemmSlots = 256;  // routed + always-on rows the prologue maps
 
 int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st);
+// The medium-problem kernel (gemm_mid.hip): whether it takes a problem (it is then the
+// faster one), and its launch.
+bool mid_gemm_takes(const GemmArgs& a, bool swiglu);
+int run_mid_gemm(const GemmArgs& a, bool swiglu, hipStream_t st);
+int num_cus();  // compute units of the current device
 
 
 // Router logits for routing = sum over n_parts partial-sum planes

@@ -46,6 +46,7 @@
 // weight rows are half gate rows (j) and half the matching up rows (I + j), so
 // silu(gate) * up is computed from fp32 accumulators held by the same lane.
 #include "dsk_internal.hpp"
+#include "gemm_common.hpp"
 #include "gemm_sched.hpp"
 #include "route_token.hpp"
 
@@ -56,9 +57,6 @@
 #include <type_traits>
 
 namespace dsk {
-
-constexpr int kMaxGroups = 128;
-constexpr int kLdsPerCU = 160 * 1024;
 
 // Tile configuration (build-time; tuned on MI355X).
 #ifndef DSK_GEMM_BM
@@ -79,24 +77,6 @@ constexpr int kLdsPerCU = 160 * 1024;
 #ifndef DSK_GEMM_STAGES
 #define DSK_GEMM_STAGES 2
 #endif
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) void global_void_t;
-
-// silu(x) = x / (1 + e^-x) with the hardware reciprocal (1 ulp), ample for a
-// result that is rounded to bf16.
-__device__ __forceinline__ float silu_f(float x) {
-  return x * __builtin_amdgcn_rcpf(1.f + __expf(-x));
-}
-
-// Reads an accumulator register where it is used: the epilogue then moves
-// the accumulators to VGPRs a few at a time instead of all at once.
-__device__ __forceinline__ float acc_read(float a) {
-  float v;
-  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
-  return v;
-}
-
 
 // Wait until at most min(ahead, MAXA) * NL vector-memory ops are pending.
 template <int MAXA, int NL>
@@ -174,13 +154,6 @@ struct GemmCfg {
   static constexpr int LDS_BYTES = RING_BYTES + ROW_TILES * BM * 4;  // dynamic LDS
 };
 
-// 16-byte slot of (row, logical chunk) in a tile of CPR-chunk LDS rows.
-template <int CPR>
-__device__ __forceinline__ int lds_swz(int row, int chunk) {
-  if constexpr (CPR == 8) return row * 8 + (chunk ^ (row & 7) ^ ((row >> 3) & 1));
-  else return row * 4 + (chunk ^ ((row >> 2) & 3));
-}
-
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool SWIGLU,
           bool GATHER, bool TILED>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel(GemmArgs p) {
@@ -240,7 +213,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
   const int per_xcd = gridDim.x >> 3;
-  const int chunk = sched_chunk(p.chunk_m_tiles, NT);
+  const int chunk = p.chunk;
   const int ntiles = sched_slot_tiles(sched_xcd_tiles(total_tiles, xcd, chunk), slot, per_xcd);
   if (ntiles == 0) return;  // uniform: no work for this workgroup
   const int nk = p.K / BK;
@@ -580,8 +553,6 @@ constexpr int kWideStageBytes = kWideBM * kWideBK * 2;  // 32 KB
 constexpr int kWideRingBytes = kWideRing * kWideStageBytes;
 constexpr int kWideRowTiles = (kLdsPerCU - kWideRingBytes - 4096) / (kWideBM * 4);
 constexpr int kWideLdsBytes = kWideRingBytes + kWideRowTiles * kWideBM * 4;
-constexpr int kRowScaleParts = 2;  // sum-of-squares partials an RMS row scale adds up
-
 
 template <bool SWIGLU, bool GATHER>
 __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs p) {
@@ -631,7 +602,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
   const int per_xcd = gridDim.x >> 3;
-  const int chunk = sched_chunk(p.chunk_m_tiles, NT);
+  const int chunk = p.chunk;
   const int ntiles = sched_slot_tiles(sched_xcd_tiles(total_tiles, xcd, chunk), slot, per_xcd);
   if (ntiles == 0) return;
   const int nk = p.K / kWideBK;  // even (K % 128 == 0, checked by the launcher)
@@ -795,22 +766,6 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
     // sit behind uniform branches. A copy of the K loop per block count would
     // merge 256 live accumulators at the branch and overflow the registers.
     const int tma = max(1, min(TM, (ct.me - ct.m0 + 31) / 32));
-    // Sum-of-squares partials of this tile's token rows (row ct.m0 + 32 i +
-    // lane % 32) for the RMS row scale, loaded now and only added up in the
-    // epilogue: a use here would make the wave wait for every DMA issued
-    // before these loads (the wait counts complete in order).
-    float rsc[TM][kRowScaleParts];
-    if constexpr (!SWIGLU && !GATHER) {
-      if (p.rowscale_ss != nullptr) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int m = min(ct.m0 + 32 * i + (lane & 31), p.M - 1);
-#pragma unroll
-          for (int q = 0; q < kRowScaleParts; ++q)
-            rsc[i][q] = p.rowscale_ss[min(q, p.rowscale_parts - 1) * p.ld_rowscale + m];
-        }
-      }
-    }
     {
       // one stage: K steps 0..3 on weight set SET; the barrier before the last
       // step publishes the next stage's tokens and frees this stage's slot
@@ -878,27 +833,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
       const int r32 = lane & 31, h = lane >> 5;
       const int col0 = SWIGLU ? ct.n0 + 32 * wave : ct.n0 + 64 * wave;  // this wave's columns
       const int rl = lane / CHUNKS, cl = lane % CHUNKS;
-      constexpr bool kRowOps = !SWIGLU && !GATHER;
-      const bool scale_rows = kRowOps && p.rowscale_ss != nullptr;
-      // whole tile inside the sum-of-squares column range (256-aligned bounds)
-      const bool sum_rows = kRowOps && p.rowsq_out != nullptr && ct.n0 >= p.rowsq_c0 &&
-                            ct.n0 < p.rowsq_c1;
-      // per-wave row partials of the sums of squares, behind the ring (the
-      // gathered kernels' row table, unused here)
-      float* s_ss = reinterpret_cast<float*>(lds + kWideRingBytes / 2);
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         if (i >= tma) continue;
-        float rs = 1.f;
-        if constexpr (kRowOps) {
-          if (scale_rows) {
-            float ss = rsc[i][0];
-#pragma unroll
-            for (int q = 1; q < kRowScaleParts; ++q)
-              if (q < p.rowscale_parts) ss += rsc[i][q];
-            rs = rsqrtf(ss * (1.f / p.rowscale_cols) + p.rowscale_eps);
-          }
-        }
 #pragma unroll
         for (int j = 0; j < JN; ++j) {
 #pragma unroll
@@ -909,7 +846,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
               if constexpr (SWIGLU)
                 v[c] = silu_f(acc_read(acc[0][i][4 * qg + c])) * acc_read(acc[1][i][4 * qg + c]);
               else
-                v[c] = acc_read(acc[j][i][4 * qg + c]) * rs;
+                v[c] = acc_read(acc[j][i][4 * qg + c]);
             }
             u32x2_t o;
             o[0] = pack_bf16x2(v[0], v[1]);
@@ -929,39 +866,10 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
           const int col = col0 + 8 * cl;
           if (m < ct.me && col < p.N)
             *reinterpret_cast<u32x4_t*>(p.C + (int64_t)m * p.ldc + col) = d;
-          if constexpr (kRowOps) {
-            if (sum_rows) {
-              // squares of the stored (bf16) values, summed over the row's 8
-              // lanes (quad swaps, then the half-row mirror)
-              float sq = 0.f;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float lo = bf16lo(d[e]), hi = bf16hi(d[e]);
-                sq = fmaf(lo, lo, sq);
-                sq = fmaf(hi, hi, sq);
-              }
-              sq += dpp_f32<0xB1>(0.f, sq);
-              sq += dpp_f32<0x4E>(0.f, sq);
-              sq += dpp_f32<0x141>(0.f, sq);
-              if (cl == 0) s_ss[wave * kWideBM + 32 * i + rr] = sq;
-            }
-          }
         }
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's staging reads done
       lds_barrier();                       // before the next DMA into the slot
-      if constexpr (kRowOps) {
-        if (sum_rows) {
-          // the tile's row sums, the four waves' column ranges added in order
-          const int t = tid;  // 256 threads, one token row each
-          const int m = ct.m0 + t;
-          if (t < 32 * tma && m < ct.me) {
-            const float ss = ((s_ss[t] + s_ss[kWideBM + t]) + s_ss[2 * kWideBM + t]) +
-                             s_ss[3 * kWideBM + t];
-            p.rowsq_out[(int64_t)((ct.n0 - p.rowsq_c0) / (64 * kWideWaves)) * p.ld_rowsq + m] = ss;
-          }
-        }
-      }
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -1404,7 +1312,7 @@ static int current_device() {
 }
 
 // CU count of the current device, queried once per device (any thread).
-static int num_cus() {
+int num_cus() {
   static std::atomic<int> cached[kMaxDevices];  // static storage: starts at 0
   const int dev = current_device();
   if (dev < 0) return 256;
@@ -1428,9 +1336,22 @@ static void allow_lds(std::once_flag (&once)[kMaxDevices], const void* kern, int
   });
 }
 
+// Chunk and workgroups of a persistent launch of at most `upper` tiles of nt N tiles
+// each. Every XCD gets a workgroup per tile it holds, up to its CUs (fewer, and 15
+// tiles in one chunk of 16 would share two workgroups of one XCD).
+static int64_t persistent_grid(GemmArgs& a, int64_t upper, int64_t nt, int row_tiles) {
+  const int64_t cus = num_cus();
+  const int bound = (int)std::min<int64_t>(upper, INT32_MAX);
+  a.chunk = a.chunk_m_tiles > 0 ? sched_chunk(a.chunk_m_tiles, (int)nt)
+                                : sched_balanced_chunk(bound, (int)cus);
+  const int64_t xcd_tiles = sched_xcd_tiles(bound, 0, a.chunk);
+  return std::max(sched_workgroups(upper, cus, row_tiles, a.chunk),
+                  std::min(kXcds * xcd_tiles, cus / kXcds * kXcds));
+}
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool SWIGLU,
           bool GATHER, bool TILED>
-static int launch_grouped_gemm(const GemmArgs& a, hipStream_t st) {
+static int launch_grouped_gemm(GemmArgs a, hipStream_t st) {
   using Cfg = GemmCfg<BM, BN, WAVES_M, WAVES_N, BK, STAGES, SWIGLU>;
   auto kern = grouped_gemm_kernel<BM, BN, WAVES_M, WAVES_N, BK, STAGES, SWIGLU, GATHER, TILED>;
   static std::once_flag once[kMaxDevices];
@@ -1439,19 +1360,18 @@ static int launch_grouped_gemm(const GemmArgs& a, hipStream_t st) {
   const int64_t nt = (a.N + Cfg::OUT_N - 1) / Cfg::OUT_N;
   // upper bound on the kernel's tile count (a group of n rows has ceil(n/BM) M tiles)
   const int64_t upper = ((int64_t)(a.M + BM - 1) / BM + (a.offsets ? G : 0)) * nt;
-  const int chunk = sched_chunk(a.chunk_m_tiles, (int)nt);
-  const int64_t nwg = sched_workgroups(upper, num_cus(), GATHER ? Cfg::ROW_TILES : 0, chunk);
+  const int64_t nwg = persistent_grid(a, upper, nt, GATHER ? Cfg::ROW_TILES : 0);
   // the gathered kernel stages every tile's row indices in an LDS table of
   // ROW_TILES tiles and computes nothing if its share is larger
   if (GATHER &&
-      (upper > INT32_MAX || sched_max_tiles((int)upper, (int)nwg, chunk) > Cfg::ROW_TILES))
+      (upper > INT32_MAX || sched_max_tiles((int)upper, (int)nwg, a.chunk) > Cfg::ROW_TILES))
     return fail(DSK_ERR_INVALID_ARG, "grouped_gemm: a workgroup's tiles exceed the LDS row table");
   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(Cfg::THREADS), Cfg::LDS_BYTES, st, a);
   return check_launch("grouped_gemm_kernel");
 }
 
 template <bool SWIGLU, bool GATHER>
-static int launch_wide_gemm(const GemmArgs& a, hipStream_t st) {
+static int launch_wide_gemm(GemmArgs a, hipStream_t st) {
   auto kern = wide_gemm_kernel<SWIGLU, GATHER>;
   static std::once_flag once[kMaxDevices];
   allow_lds(once, reinterpret_cast<const void*>(kern), kWideLdsBytes);
@@ -1459,10 +1379,9 @@ static int launch_wide_gemm(const GemmArgs& a, hipStream_t st) {
   const int G = a.offsets != nullptr ? a.G : 1;
   const int64_t nt = (a.N + OUT_N - 1) / OUT_N;
   const int64_t upper = ((int64_t)(a.M + kWideBM - 1) / kWideBM + (a.offsets ? G : 0)) * nt;
-  const int chunk = sched_chunk(a.chunk_m_tiles, (int)nt);
-  const int64_t nwg = sched_workgroups(upper, num_cus(), GATHER ? kWideRowTiles : 0, chunk);
+  const int64_t nwg = persistent_grid(a, upper, nt, GATHER ? kWideRowTiles : 0);
   if (GATHER &&
-      (upper > INT32_MAX || sched_max_tiles((int)upper, (int)nwg, chunk) > kWideRowTiles))
+      (upper > INT32_MAX || sched_max_tiles((int)upper, (int)nwg, a.chunk) > kWideRowTiles))
     return fail(DSK_ERR_INVALID_ARG, "wide_gemm: a workgroup's tiles exceed the LDS row table");
   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(64 * kWideWaves), kWideLdsBytes, st, a);
   return check_launch("wide_gemm_kernel");
@@ -1548,7 +1467,8 @@ static int validate_gemm(const GemmArgs& a, const char* who) {
 }
 
 // Kernel choice: groups known to hold at most 64 rows (decode) go to the
-// weight-streaming kernel, everything else to the 256 x 256 tile kernel.
+// weight-streaming kernel, then whatever the medium-problem kernel takes
+// (gemm_mid.hip), everything else to the 256 x 256 tile kernels.
 template <bool SWIGLU, bool GATHER, bool TILED>
 static int run_gemm_t(const GemmArgs& a, hipStream_t st) {
   // groups of at most 64 rows (decode): weight streaming kernel
@@ -1559,6 +1479,7 @@ static int run_gemm_t(const GemmArgs& a, hipStream_t st) {
                    a.rt_T >= 1 && a.rt_T <= kRouteInGemmTokens && a.M <= kRouteInGemmSlots),
               DSK_ERR_INVALID_ARG, "grouped GEMM: routing in the prologue needs a small SwiGLU step");
   if (rows <= kSkinnyMaxRows) return launch_skinny<SWIGLU, GATHER, TILED>(a, rows, st);
+  if (mid_gemm_takes(a, SWIGLU)) return run_mid_gemm(a, SWIGLU, st);
 #ifndef DSK_GEMM_WIDE
 #define DSK_GEMM_WIDE 1
 #endif
@@ -1579,9 +1500,9 @@ static int run_gemm_t(const GemmArgs& a, hipStream_t st) {
 int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
   if (a.M == 0) return DSK_OK;
   if (a.rowsq_out != nullptr || a.rowscale_ss != nullptr) {
-    // row statistics live in the one-wave-per-SIMD kernel's epilogue only
+    // row statistics live in the medium-problem kernel's epilogue only
     DSK_REQUIRE(a.b_tiled && !swiglu && a.a_rows == nullptr && a.offsets == nullptr &&
-                    a.K % (2 * kWideBK) == 0 && aligned16(a.C) && a.ldc % 8 == 0,
+                    a.K % 128 == 0 && aligned16(a.C) && a.ldc % 8 == 0,
                 DSK_ERR_INVALID_ARG,
                 "linear row statistics: need a tiled weight, K % 128 == 0 and 16-byte aligned "
                 "output rows");
@@ -1592,11 +1513,11 @@ int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
                 "linear_rowsq: the column range must be 256-aligned inside [0, N) and "
                 "ld_rowsq >= M");
     DSK_REQUIRE(a.rowscale_ss == nullptr ||
-                    (a.rowscale_parts >= 1 && a.rowscale_parts <= kRowScaleParts &&
+                    (a.rowscale_parts >= 1 && a.rowscale_parts <= 2 &&
                      a.rowscale_cols > 0 && a.ld_rowscale >= a.M),
                 DSK_ERR_INVALID_ARG,
                 "linear_rowscale: need 1 or 2 parts, cols > 0 and ld_rowscale >= M");
-    return launch_wide_gemm<false, false>(a, st);
+    return run_mid_gemm(a, false, st);
   }
   const bool g = a.a_rows != nullptr;
   if (a.b_tiled) {

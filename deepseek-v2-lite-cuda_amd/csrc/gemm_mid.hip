@@ -1,0 +1,370 @@
+// Grouped GEMM for medium problems (gfx950): tiles of 64 or 128 token rows, two or
+// more workgroups per CU. It runs the shapes that lie between the weight-streaming
+// kernel (groups of at most 64 rows) and the 256 x 256 tile kernels (several rounds
+// of full tiles): the expert GEMMs of a few hundred tokens, where a 256-row tile is
+// mostly padding, and dense projections whose 256 x 256 tiles do not cover the CUs.
+//
+// Data path, as in the one-wave-per-SIMD kernel (gemm.hip): a wave owns TN blocks of
+// 32 weight rows against every token row of the tile. Its weight fragments go from
+// memory straight into registers, two stages of 64 K ahead (nobody else needs them);
+// the token rows go through a 4-deep LDS ring filled by global->LDS DMA three stages
+// ahead and are read back by all 4 waves. One barrier per stage. A workgroup runs
+// one tile; several share a CU, so one's prologue, epilogue and waits are covered by
+// another's loads and MFMAs, without a persistent stage stream.
+//
+// The order of memory operations per stage is fixed (TM DMA instructions, then TN
+// weight loads per K step), which the explicit vmcnt waits count on; past the end of
+// K the last stage is repeated into slots and registers that nobody reads again.
+#include "dsk_internal.hpp"
+#include "gemm_common.hpp"
+#include "gemm_sched.hpp"
+
+#include <type_traits>
+
+namespace dsk {
+
+constexpr int kMidWaves = 4;
+constexpr int kMidThreads = 64 * kMidWaves;
+constexpr int kMidBK = 64;
+constexpr int kMidRing = 4;
+
+template <int TM, int TN, bool SWIGLU, bool GATHER, bool TILED>
+__global__ __launch_bounds__(kMidThreads, 2) void mid_gemm_kernel(GemmArgs p, int chunk) {
+  static_assert(TM == 2 || TM == 4, "64 or 128 token rows per tile");
+  static_assert(TN == 1 || TN == 2, "one or two weight blocks per wave");
+  static_assert(!SWIGLU || TN == 2, "SwiGLU pairs a gate and an up block");
+  constexpr int BM = 32 * TM;
+  constexpr int OUT_N = SWIGLU ? 32 * kMidWaves : 32 * TN * kMidWaves;
+  constexpr int KSTEPS = kMidBK / 16;
+  constexpr int kStageBytes = BM * kMidBK * 2;
+  __shared__ __attribute__((aligned(1024))) char s_ring[kMidRing * kStageBytes];
+  __shared__ int s_inc[kMaxGroups];
+  __shared__ int s_mb[kMaxGroups];
+  __shared__ int s_me[kMaxGroups];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int NT = (p.N + OUT_N - 1) / OUT_N;
+  // ---- group table: row ranges and inclusive prefix of tile counts
+  int total = (p.M + BM - 1) / BM * NT;
+  if (p.offsets != nullptr) {
+    if (tid < kMaxGroups) {
+      int cnt = 0;
+      if (tid < p.G) {
+        const int lo = min(max(p.offsets[tid], 0), p.M);
+        const int hi = min(max(p.offsets[tid + 1], lo), p.M);
+        s_mb[tid] = lo;
+        s_me[tid] = hi;
+        cnt = ((hi - lo + BM - 1) / BM) * NT;
+      }
+      s_inc[tid] = wave_inclusive_scan(cnt);
+    }
+    __syncthreads();
+    const int carry = s_inc[63];
+    __syncthreads();
+    if (tid >= 64 && tid < kMaxGroups) s_inc[tid] += carry;
+    __syncthreads();
+    total = s_inc[p.G - 1];
+  }
+  // one tile per workgroup, dealt to the XCDs in chunks (gemm_sched.hpp); the grid
+  // covers every tile of non-decreasing offsets
+  const int W = sched_tile_index(blockIdx.x & 7, blockIdx.x >> 3, 0, 1, chunk);
+  if (W >= total) return;  // uniform
+
+  // ---- the tile: group g, rows [m0, me), output columns from n0
+  int g = 0, mb = 0, gme = p.M, local = W;
+  if (p.offsets != nullptr) {
+    int lo = 0, hi = p.G - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (s_inc[mid] > W) hi = mid; else lo = mid + 1;
+    }
+    g = __builtin_amdgcn_readfirstlane(lo);
+    local = W - (g > 0 ? s_inc[g - 1] : 0);
+    mb = s_mb[g];
+    gme = s_me[g];
+  }
+  const int mt = (gme - mb + BM - 1) / BM;
+  const int nblk = (gme - mb + 31) / 32;
+  int nt, mi;
+  sched_group_tile(local, mt, NT, &nt, &mi);
+  nt = __builtin_amdgcn_readfirstlane(nt);
+  const int m0 = __builtin_amdgcn_readfirstlane(mb + 32 * (mi * nblk / mt));
+  const int me = __builtin_amdgcn_readfirstlane(min(mb + 32 * ((mi + 1) * nblk / mt), gme));
+  const int n0 = nt * OUT_N;
+  const int tma = (me - m0 + 31) / 32;  // token blocks with rows
+  const int nk = p.K / kMidBK;
+
+  // ---- weight fragments of this wave: byte offset of block j at k = 0
+  const char* Bg = reinterpret_cast<const char*>(p.B + (int64_t)g * p.b_group_stride);
+  uint32_t b_off[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int last = p.N / 32 - 1;
+    int rb;
+    if constexpr (SWIGLU) {
+      const int ob = min(n0 / 32 + wave, last);
+      rb = j == 0 ? ob : p.up_row_offset / 32 + ob;  // gate rows, then up rows
+    } else {
+      rb = min(n0 / 32 + TN * wave + j, last);
+    }
+    if constexpr (TILED)
+      b_off[j] = (uint32_t)((((int64_t)rb * (p.K / 16)) * 512 + lane * 8) * 2);
+    else
+      b_off[j] = (uint32_t)(((int64_t)(32 * rb + (lane & 31)) * p.ldb + 8 * (lane >> 5)) * 2);
+  }
+  auto issue_b = [&](bf16x8_t (&dst)[TN], int stage, int k) __attribute__((always_inline)) {
+    const uint32_t koff = (uint32_t)(min(stage, nk - 1) * KSTEPS + k) * (TILED ? 1024 : 32);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) dst[j] = *reinterpret_cast<const bf16x8_t*>(Bg + (b_off[j] + koff));
+  };
+
+  // ---- token DMA: instruction i of a wave moves rows 8 (wave + 4 i) .. + 7 of the
+  // tile (128 bytes each, chunk-swizzled); rows past the tile repeat its first row
+  const char* Abase = reinterpret_cast<const char*>(p.A);
+  const int dma_row = lane >> 3;
+  const int dma_chunk = (lane & 7) ^ dma_row ^ (wave & 1);
+  const int row_limit = GATHER ? p.a_rows_limit : p.M;
+  uint32_t a_off[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + 8 * (wave + kMidWaves * i) + dma_row;
+    int row = m < me ? m : m0;
+    if constexpr (GATHER) row = p.a_rows[row];
+    row = (row >= 0 && row < row_limit) ? row : 0;
+    a_off[i] = (uint32_t)(((int64_t)row * p.lda + dma_chunk * 8) * 2);
+  }
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_ring));
+  auto issue_a = [&](int stage) __attribute__((always_inline)) {
+    const uint32_t koff = (uint32_t)min(stage, nk - 1) * kMidBK * 2;
+    const uint32_t dst = lds_base + (stage % kMidRing) * kStageBytes;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      dma_1kb(Abase, a_off[i] + koff, dst + (wave + kMidWaves * i) * 1024);
+  };
+
+  bf16x8_t fb[2][KSTEPS][TN];  // weight fragments, register set = stage parity
+  bf16x8_t fa[2][TM];          // token fragments, double-buffered by K step
+  floatx16_t acc[TN][TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.f;
+  const u32x4_t* lds4 = reinterpret_cast<const u32x4_t*>(s_ring);
+  auto read_a = [&](bf16x8_t (&dst)[TM], int slot, int kk) __attribute__((always_inline)) {
+    const u32x4_t* As = lds4 + slot * (kStageBytes / 16);
+    const int ch = 2 * kk + (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      dst[i] = __builtin_bit_cast(bf16x8_t, As[lds_swz<8>(32 * i + (lane & 31), ch)]);
+  };
+
+  // ---- prologue: A0 B0 A1 B1 A2 in flight, A0 landed
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    issue_a(s);
+    if (s < 2) {
+#pragma unroll
+      for (int k = 0; k < KSTEPS; ++k) issue_b(fb[s][k], s, k);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  wait_vmcnt<2 * TM + 2 * KSTEPS * TN>();  // A0 done; B0 A1 B1 A2 may be pending
+  lds_barrier();
+  read_a(fa[0], 0, 0);
+
+  auto stage = [&](auto set_c, int s) __attribute__((always_inline)) {
+    constexpr int SET = decltype(set_c)::value;
+    issue_a(s + 3);  // into the slot of stage s - 1, which every wave has read
+#pragma unroll
+    for (int k = 0; k < KSTEPS; ++k) {
+      if (k == KSTEPS - 1) {
+        // A(s + 1) has landed: after it came at least B(s) or B(s + 1) (4 TN), A(s + 2),
+        // A(s + 3) and 3 TN loads of B(s + 2)
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<2 * TM + 7 * TN>();
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): own LDS reads done
+        lds_barrier();
+        read_a(fa[(k + 1) & 1], (s + 1) % kMidRing, 0);
+      } else {
+        read_a(fa[(k + 1) & 1], s % kMidRing, k + 1);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if (i < TM / 2 || i < tma) {  // uniform
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[SET][k][j], fa[k & 1][i],
+                                                                acc[j][i], 0, 0, 0);
+        }
+      }
+      issue_b(fb[SET][k], s + 2, k);
+    }
+  };
+#pragma unroll 1
+  for (int s = 0; s < nk; s += 2) {
+    stage(std::integral_constant<int, 0>{}, s);
+    if (s + 1 < nk) stage(std::integral_constant<int, 1>{}, s + 1);
+  }
+
+  // ---- epilogue through the LDS: each wave stages one 32-row block at a time and
+  // stores whole row segments (64 or 128 bytes)
+  wait_vmcnt<0>();  // no DMA lands in the ring any more
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  lds_barrier();
+  constexpr int JN = SWIGLU ? 1 : TN;
+  constexpr int ROW_BYTES = 64 * JN;
+  constexpr int CHUNKS = ROW_BYTES / 16;
+  constexpr int ROWS_PER_INST = 64 / CHUNKS;
+  auto swz = [](int row) { return JN == 1 ? (row >> 2) & 3 : (row >> 1) & 7; };
+  char* st = s_ring + wave * 4096;
+  const int r32 = lane & 31, h = lane >> 5;
+  const int col0 = n0 + 32 * JN * wave;
+  const int rl = lane / CHUNKS, cl = lane % CHUNKS;
+  // row statistics (GemmArgs): whole 256-column tiles, TN = 2 only
+  constexpr bool kRowOps = !SWIGLU && !GATHER && TILED && TN == 2;
+  const bool scale_rows = kRowOps && p.rowscale_ss != nullptr;
+  const bool sum_rows = kRowOps && p.rowsq_out != nullptr && n0 >= p.rowsq_c0 && n0 < p.rowsq_c1;
+  float* s_ss = reinterpret_cast<float*>(s_ring + kMidWaves * 4096);  // [wave][row of the tile]
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    if (i >= tma) continue;
+    float rs = 1.f;
+    if constexpr (kRowOps) {
+      if (scale_rows) {
+        const int m = min(m0 + 32 * i + r32, p.M - 1);
+        float ss = p.rowscale_ss[m];
+        for (int q = 1; q < p.rowscale_parts; ++q) ss += p.rowscale_ss[q * p.ld_rowscale + m];
+        rs = rsqrtf(ss * (1.f / p.rowscale_cols) + p.rowscale_eps);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+#pragma unroll
+      for (int qg = 0; qg < 4; ++qg) {
+        float v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if constexpr (SWIGLU) v[c] = silu_f(acc[0][i][4 * qg + c]) * acc[1][i][4 * qg + c];
+          else if constexpr (kRowOps) v[c] = acc[j][i][4 * qg + c] * rs;
+          else v[c] = acc[j][i][4 * qg + c];
+        }
+        u32x2_t o;
+        o[0] = pack_bf16x2(v[0], v[1]);
+        o[1] = pack_bf16x2(v[2], v[3]);
+        const int ch = 4 * j + qg;
+        *reinterpret_cast<u32x2_t*>(st + r32 * ROW_BYTES + ((ch ^ swz(r32)) * 16) +
+                                    ((h ^ ((r32 >> 4) & 1)) * 8)) = o;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 32 / ROWS_PER_INST; ++q) {
+      const int rr = q * ROWS_PER_INST + rl;
+      u32x4_t d = *reinterpret_cast<const u32x4_t*>(st + rr * ROW_BYTES + ((cl ^ swz(rr)) * 16));
+      if ((rr >> 4) & 1) d = u32x4_t{d[2], d[3], d[0], d[1]};  // halves were swapped
+      const int m = m0 + 32 * i + rr;
+      const int col = col0 + 8 * cl;
+      if (m < me && col < p.N) *reinterpret_cast<u32x4_t*>(p.C + (int64_t)m * p.ldc + col) = d;
+      if constexpr (kRowOps) {
+        if (sum_rows) {
+          // squares of the stored (bf16) values, summed over the row's 8 lanes
+          // (quad swaps, then the half-row mirror)
+          float sq = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float lo = bf16lo(d[e]), hi = bf16hi(d[e]);
+            sq = fmaf(lo, lo, sq);
+            sq = fmaf(hi, hi, sq);
+          }
+          sq += dpp_f32<0xB1>(0.f, sq);
+          sq += dpp_f32<0x4E>(0.f, sq);
+          sq += dpp_f32<0x141>(0.f, sq);
+          if (cl == 0) s_ss[wave * BM + 32 * i + rr] = sq;
+        }
+      }
+    }
+  }
+  if constexpr (kRowOps) {
+    if (sum_rows) {
+      __syncthreads();
+      // the tile's row sums, the four waves' column ranges added in order
+      if (tid < 32 * tma && m0 + tid < me) {
+        const float ss = ((s_ss[tid] + s_ss[BM + tid]) + s_ss[2 * BM + tid]) + s_ss[3 * BM + tid];
+        p.rowsq_out[(int64_t)((n0 - p.rowsq_c0) / OUT_N) * p.ld_rowsq + m0 + tid] = ss;
+      }
+    }
+  }
+}
+
+template <int TM, int TN, bool SWIGLU, bool GATHER, bool TILED>
+static int launch_mid(const GemmArgs& a, hipStream_t st) {
+  constexpr int OUT_N = SWIGLU ? 32 * kMidWaves : 32 * TN * kMidWaves;
+  const int64_t nt = (a.N + OUT_N - 1) / OUT_N;
+  const int64_t tiles =
+      ((int64_t)(a.M + 32 * TM - 1) / (32 * TM) + (a.offsets != nullptr ? a.G : 0)) * nt;
+  if (tiles > INT32_MAX / 2)
+    return fail(DSK_ERR_INVALID_ARG, "mid_gemm: too many tiles");
+  const int chunk = sched_balanced_chunk((int)tiles, num_cus());
+  const int64_t grid = (tiles + kXcds * chunk - 1) / (kXcds * chunk) * (kXcds * chunk);
+  hipLaunchKernelGGL((mid_gemm_kernel<TM, TN, SWIGLU, GATHER, TILED>), dim3((unsigned)grid),
+                     dim3(kMidThreads), 0, st, a, chunk);
+  return check_launch("mid_gemm_kernel");
+}
+
+bool mid_gemm_takes(const GemmArgs& a, bool swiglu) {
+  const bool gather = a.a_rows != nullptr, grouped = a.offsets != nullptr;
+  if (a.N % 32 || a.up_row_offset % 32 || !aligned16(a.C) || a.ldc % 8) return false;
+  if (a.a_group_stride || a.c_group_stride || a.C2 != nullptr) return false;
+  if (!grouped) return !swiglu && !gather;
+  if (!a.offsets_sorted) return false;  // overlapping groups can make more tiles than the grid
+  // Grouped: tiled weights in the fused layer's two forms. Measured on MI355X in the
+  // MoE layer (64 experts top-6 and 2 always-on groups, T tokens, M / G = 0.12 T;
+  // this kernel against the 256 x 256 ones, us):
+  //   GEMM1  T = 250 138 / 163, 600 159 / 193, 1000 164 / 207, 2000 224 / 231,
+  //          3000 316 / 332, 4096 381 / 371, 8192 695 / 677
+  //   GEMM2  T = 250 76 / 108, 600 87 / 109, 1000 107 / 114, 1400 117 / 121,
+  //          2000 133 / 133, 3000 187 / 185, 4096 221 / 217
+  // With row-major weights a fragment load touches 32 rows, and the DMA of the 256 x 256
+  // kernel wins (T = 600: 358 against 318 us for both).
+  const int64_t avg = a.M / (a.G > 0 ? a.G : 1);
+  return a.b_tiled && swiglu == gather && avg <= (swiglu ? 430 : 230);
+}
+
+int run_mid_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
+  if (swiglu) return launch_mid<4, 2, true, true, true>(a, st);
+  if (a.offsets != nullptr) {
+    // few rows per group: 64-row tiles, and half the weight rows per workgroup, which
+    // spreads the weight stream over twice the workgroups (T = 250: 76 us against 91)
+    if (a.M / (a.G > 0 ? a.G : 1) <= 80) return launch_mid<2, 1, false, false, true>(a, st);
+    return launch_mid<4, 2, false, false, true>(a, st);
+  }
+  // Dense: the tile with the least estimated time, tiles on the fullest CU times the
+  // cost of one tile. The costs are proportional to what a tile took at K = 2048 with
+  // one tile per CU (64 x 128 tokens x weight rows 13 us, 64 x 256 17.5, 128 x 256 27);
+  // over M = 65..8192 and the layer's three (N, K) the choice was the fastest of them or
+  // within 6 % of it. Measured against the 256 x 256 kernel:
+  // N = 2048, K = 2048: M = 257 15 / 282 us, 1111 19 / 166, 4096 36 / 54, 8192 61 / 70;
+  // N = 3648: M = 1111 30 / 89, 4096 62 / 101, 16384 228 / 242; N = 4096, K = 512:
+  // M = 1111 12.5 / 34, 16384 81 / 87.
+  const int64_t cus = num_cus();
+  auto cost = [&](int bm, int bn, double per_tile) {
+    const int64_t t = (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+    return (double)((t + cus - 1) / cus) * per_tile;
+  };
+  const bool row_stats = a.rowsq_out != nullptr || a.rowscale_ss != nullptr;  // whole 256 columns
+  const double c64w = cost(64, 256, 17.5), c128w = cost(128, 256, 27.0);
+  const double wide = c64w < c128w ? c64w : c128w;
+  if (!row_stats && cost(64, 128, 13.0) < wide)
+    return a.b_tiled ? launch_mid<2, 1, false, false, true>(a, st)
+                     : launch_mid<2, 1, false, false, false>(a, st);
+  if (c64w < c128w)
+    return a.b_tiled ? launch_mid<2, 2, false, false, true>(a, st)
+                     : launch_mid<2, 2, false, false, false>(a, st);
+  return a.b_tiled ? launch_mid<4, 2, false, false, true>(a, st)
+                   : launch_mid<4, 2, false, false, false>(a, st);
+}
+
+}  // namespace dsk

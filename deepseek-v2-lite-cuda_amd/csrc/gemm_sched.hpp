@@ -36,6 +36,19 @@ DSK_HD int sched_chunk(int chunk_m_tiles, int nt) {
   return chunk_m_tiles > 0 ? chunk_m_tiles * nt : kTileChunk;
 }
 
+// Chunk for a launch of `total` tiles on `cus` compute units: the largest of 16, 8, 4,
+// 2, 1 that leaves no XCD with more tiles per CU than an even deal would (a chunk of
+// 16 on 15 tiles would run all of them on one XCD).
+DSK_HD int sched_xcd_tiles(int total, int xcd, int chunk);
+DSK_HD int sched_balanced_chunk(int total, int cus) {
+  const int per_xcd = cus / kXcds > 0 ? cus / kXcds : 1;
+  const int even = (total + kXcds - 1) / kXcds;  // tiles of the fullest XCD at chunk 1
+  const int rounds = (even + per_xcd - 1) / per_xcd;
+  for (int chunk = kTileChunk; chunk > 1; chunk /= 2)
+    if (sched_xcd_tiles(total, 0, chunk) <= rounds * per_xcd) return chunk;
+  return 1;
+}
+
 // Tiles held by XCD `xcd` out of `total`.
 DSK_HD int sched_xcd_tiles(int total, int xcd, int chunk) {
   const int n_chunks = (total + chunk - 1) / chunk;

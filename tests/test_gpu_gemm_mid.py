@@ -1,0 +1,91 @@
+"""The medium-problem GEMM kernel (csrc/gemm_mid.hip) at the edges of its tiles.
+
+Bound per output: the bf16 rounding of the result (8 significant bits: 2^-8 |y|) and the
+fp32 accumulation, at most K 2^-23 sum_k |x_k w_k| (one rounding per term, any order)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def dsk():
+    import ds_kernels
+    return ds_kernels
+
+
+def _check(out, x, w, scale=None):
+    xd, wd = x.double(), w.double()
+    ref, room = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    if scale is not None:
+        ref, room = ref * scale, room * scale
+    err = (out.double() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + x.shape[1] * 2.0 ** -23 * room).all()), float(err.max())
+
+
+# 64 x 128, 64 x 256 and 128 x 256 tiles (by the rule: few tiles, more than a CU each, large),
+# one row past a tile, one short of it, widths of one block and of a partial tile, odd
+# numbers of 64-K stages
+@pytest.mark.parametrize("M,N,K", [
+    (65, 32, 64), (127, 96, 192), (128, 160, 128), (129, 2048, 2048), (200, 3648, 64),
+    (777, 3648, 2048), (1000, 4096, 512), (1111, 3648, 2048), (2049, 2080, 1408),
+    (4097, 4096, 512)])
+def test_dense(dsk, M, N, K):
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K + 64, generator=g).to(torch.bfloat16).to(DEV)[:, :K]   # strided rows
+    w = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    tiled = dsk.linear(x, dsk.tile_weights(w[None])[0])
+    _check(tiled, x, w)
+    assert torch.equal(tiled, dsk.linear(x, w))          # row-major weight: the same sums
+    guard = torch.full((M + 2, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    dsk.linear(x, dsk.tile_weights(w[None])[0], out=guard[1:M + 1, :N])
+    assert torch.equal(guard[1:M + 1, :N], tiled)
+    assert bool((guard[0] == 7).all() and (guard[M + 1] == 7).all() and (guard[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("M", [1, 33, 64, 200, 777, 1111, 4100])
+def test_row_statistics(dsk, M):
+    """linear_rowsq / linear_rowscale on 64- and 128-row tiles."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, 256, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(800, 256, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    wt = dsk.tile_weights(w[None])[0]
+    y, ss = dsk.linear_rowsq(x, wt, 256, 768)
+    _check(y, x, w)
+    ref = y[:, 256:768].double().square().view(M, 2, 256).sum(-1).t()
+    assert bool(((ss.double() - ref).abs() <= 256 * 2.0 ** -23 * ref).all())
+    z = dsk.linear_rowscale(x, wt, ss, 512, 1e-6)
+    r = torch.rsqrt(ss.double().sum(0) / 512 + 1e-6)[:, None]
+    _check(z, x, w, r * (1 + 2.0 ** -20))
+
+
+@pytest.mark.parametrize("T,bias", [(65, 0.0), (150, 3.0), (600, 0.0), (600, 6.0), (1400, 3.0),
+                                    (3000, 0.0)])
+def test_fused_layer_groups(dsk, T, bias):
+    """The grouped forms in the fused layer: equal and very unequal groups (some empty, some
+    of nearly T rows) against per-expert products of the routing it returns."""
+    E, K, H, I, nsh = 16, 4, 256, 192, 2
+    g = torch.Generator().manual_seed(T)
+    rnd = lambda *s, std=0.08: (torch.randn(*s, generator=g) * std).to(torch.bfloat16).to(DEV)  # noqa: E731
+    x, wg = rnd(T, H, std=1.0), rnd(E, H)
+    w1, w2 = rnd(E + nsh, 2 * I, H), rnd(E + nsh, H, I)
+    logits = (x.float() @ wg.float().t()
+              - bias * torch.log(torch.arange(1.0, E + 1)).to(DEV)).contiguous()
+    out, (idx, wt, off) = dsk.moe_fused_forward_logits(
+        logits, x, dsk.tile_weights(w1), dsk.tile_weights(w2), K, nsh, E, return_routing=True)
+    ref = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(E + nsh):
+        t, k = (idx == e).nonzero(as_tuple=True) if e < E else (torch.arange(T, device=DEV), None)
+        h = x[t].double() @ w1[e].double().t()
+        h = torch.nn.functional.silu(h[:, :I]) * h[:, I:]
+        y = h @ w2[e].double().t()
+        ref.index_add_(0, t, y if k is None else y * wt[t, k].double()[:, None])
+    counts = (off[1:] - off[:-1]).cpu().numpy()
+    np.testing.assert_array_equal(counts, np.bincount(idx.cpu().numpy().ravel(), minlength=E))
+    # bf16 h, y and out: three roundings of 2^-8 on sums that add in quadrature
+    err = (out.double() - ref).norm() / ref.norm()
+    assert float(err) <= 2.0 ** -7, float(err)
+    assert torch.equal(out, dsk.moe_fused_forward_logits(
+        logits, x, dsk.tile_weights(w1), dsk.tile_weights(w2), K, nsh, E))
