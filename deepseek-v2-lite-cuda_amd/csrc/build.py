@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 DEFAULT_OUT = os.path.join(PKG, "ds_kernels", "libdsk.so")
 SOURCES = ["dsk_errors.hip", "gate.hip", "moe_route.hip", "gemm.hip", "gemm_mid.hip", "gemv.hip", "mla.hip", "mla_decode.hip",
-           "mla_prefill.hip", "moe_layer.hip"]
+           "mla_prefill.hip", "mla_layer.hip", "moe_layer.hip"]
 
 
 def hipcc() -> str:

@@ -60,6 +60,12 @@ SIGNATURES = {
     "dsk_mla_prefill_attention": (_I, [_P, _I64, _P, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _F,
                                        _I, _P, _I, _I64, _I64, _I64, _P, _I64, _I, _I, _I, _I,
                                        _P]),
+    "dsk_mla_forward_workspace_size": (_SZ, [_I, _I, _I]),
+    "dsk_mla_forward": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _F, _F, _I, _P, _I, _I64, _I64,
+                             _I64, _P, _I, _I, _I, _I, _P, _SZ, _P]),
+    "dsk_mla_decode_forward_workspace_size": (_SZ, [_I, _I, _I]),
+    "dsk_mla_decode_forward": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _F, _F, _I, _I,
+                                    _I, _I, _I, _P, _P, _SZ, _P]),
     "dsk_rms_norm": (_I, [_P, _I64, _P, _P, _I64, _I, _I, _F, _P]),
     "dsk_rms_norm_f32": (_I, [_P, _I64, _P, _P, _I64, _I, _I, _F, _P]),
     "dsk_rope": (_I, [_P, _I64, _I64, _I64, _P, _P, _I64, _I64, _P, _I, _I, _I, _I, _P]),
@@ -100,6 +106,25 @@ def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib.dsk_last_error().decode(errors="replace")
         raise DskError(f"{what} failed (status {rc}): {msg}")
+
+
+class _NoGuard:
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NO_GUARD = _NoGuard()
+
+
+def on_device(device: torch.device):
+    """Context in which `device` is current; nothing to do when it already is (a
+    torch.cuda.device context costs ~3 us of host time per op)."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _NO_GUARD
+    return torch.cuda.device(device)
 
 
 def stream_handle(device: torch.device) -> int:

@@ -21,6 +21,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import ops
+from ._lib import check, lib, on_device, stream_handle
 from .expert_prepack import pack_tensors, tile_weights
 from .moe_fused import moe_layer_forward
 
@@ -192,6 +193,12 @@ def rope_tables_for(cos: torch.Tensor, sin: torch.Tensor, s: int,
     return cs[pid].contiguous(), sn[pid].contiguous()
 
 
+def is_tiled(w: Optional[torch.Tensor], shape: tuple, device: torch.device) -> bool:
+    """Whether w is a fragment-tiled bf16 weight (stack) of the logical shape on device."""
+    return (w is not None and w.shape == (*shape[:-2], shape[-2] // 32, shape[-1] // 16, 64, 8)
+            and w.dtype == torch.bfloat16 and w.device == device and w.is_contiguous())
+
+
 def mla_forward(x: torch.Tensor, W: MLAWeights, cos: torch.Tensor, sin: torch.Tensor,
                 eps: float = 1e-6, attention_mask: Optional[torch.Tensor] = None,
                 position_ids: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -207,7 +214,14 @@ def mla_forward(x: torch.Tensor, W: MLAWeights, cos: torch.Tensor, sin: torch.Te
     b, s, H = x.shape
     h, r = W.n_heads, W.rope_dim
     cs, sn = rope_tables_for(cos, sin, s, position_ids)
-    if (W.nope, r, W.v_dim) == (128, 64, 128):
+    dims = (W.nope, r, W.v_dim, W.kv_lora)
+    if (dims == (128, 64, 128, 512) and h % 4 == 0 and x.is_cuda and x.dtype == torch.bfloat16
+            and is_tiled(W.q_kva, (h * 192 + 576, H), x.device)
+            and is_tiled(W.kvb_w, (h * 256, 512), x.device)
+            and is_tiled(W.o, (H, h * 128), x.device)):
+        return _mla_forward_native(x.contiguous(), W, cs.contiguous(), sn.contiguous(), eps,
+                                   attention_mask)
+    if dims[:3] == (128, 64, 128):
         qr, kv, kva, _ = _projection_rows(x, W, eps, with_latent=False)
         cs, sn = cs.contiguous(), sn.contiguous()
         ct, st = ((t if t.dim() == 3 else t[None])[:, None].expand(b, 1, s, r) for t in (cs, sn))
@@ -225,6 +239,34 @@ def mla_forward(x: torch.Tensor, W: MLAWeights, cos: torch.Tensor, sin: torch.Te
     o = torch.matmul(p, v)                                             # [b,h,s,v]
     o = o.transpose(1, 2).reshape(b, s, W.n_heads * W.v_dim)
     return ops.linear(o, W.o)
+
+
+def _mla_forward_native(x, W: MLAWeights, cs, sn, eps, attention_mask):
+    """mla_forward on tiled weights in one C call (dsk_mla_forward): the same kernels, with
+    the latent norm in the projections' epilogues, the intermediates in one workspace."""
+    op = "mla_forward"
+    b, s, H = x.shape
+    h, dev = W.n_heads, x.device
+    ops._req(cs.shape == sn.shape and cs.shape[-2:] == (s, 64) and cs.shape[:-2] in ((), (b,))
+             and cs.device == dev and sn.device == dev,
+             f"{op}: cos/sin must be [>= {s}, 64] or [{b}, >= {s}, 64] on x's device.")
+    m = (ops._expand_mask(op, attention_mask, dev, b, h, s, s)
+         if attention_mask is not None else None)
+    out = torch.empty_like(x)
+    if out.numel() == 0:
+        return out
+    ws = torch.empty(lib.dsk_mla_forward_workspace_size(b, s, h), dtype=torch.uint8, device=dev)
+    mptr, mkind, msb, msh, msq = None, 0, 0, 0, 0
+    if m is not None:
+        mptr, mkind = m.data_ptr(), 1 if m.dtype == torch.float32 else 0
+        msb, msh, msq = m.stride(0), m.stride(1), m.stride(2)
+    with on_device(dev):
+        check(lib.dsk_mla_forward(
+            x.data_ptr(), W.q_kva.data_ptr(), W.kvb_w.data_ptr(), W.o.data_ptr(), cs.data_ptr(),
+            sn.data_ptr(), 64, s * 64 if cs.dim() == 3 else 0, eps, W.softmax_scale,
+            1 if m is None else 0, mptr, mkind, msb, msh, msq, out.data_ptr(), b, s, h, H,
+            ws.data_ptr(), ws.numel(), stream_handle(dev)), op)
+    return out
 
 
 def _assemble_attention_operands(x, W: MLAWeights, cs, sn, eps, sp):

@@ -27,8 +27,9 @@ from typing import Optional, Tuple
 import torch
 
 from . import ops
+from ._lib import check, lib, on_device, stream_handle
 from .expert_prepack import tile_weights, untile_weights
-from .mla import MLAWeights
+from .mla import MLAWeights, is_tiled
 
 
 class LatentKVCache:
@@ -205,10 +206,8 @@ class AbsorbedMLAWeights:
 # once per new token, which a long step cannot amortise.
 UP_PROJECTED_MIN_TOKENS = 128
 
-# Decode steps of at most this many tokens run their projections on the
-# vector-ALU row kernel (dsk_linear_rows); longer ones on the small-group MFMA
-# kernel.
-ROWS_MAX_TOKENS = 4
+# Largest decode step (new tokens of all sequences) that runs as one C call.
+NATIVE_MAX_TOKENS = 64
 
 
 def _attend_up_projected(q: torch.Tensor, cache: LatentKVCache, W: MLAWeights, cos: torch.Tensor,
@@ -300,36 +299,28 @@ def _decode_step(x: torch.Tensor, W: MLAWeights, cache: LatentKVCache, rows: tor
     b, n, H = x.shape
     h, nope, r, vd, lora = W.n_heads, W.nope, W.rope_dim, W.v_dim, W.kv_lora
     T = b * n
+    if ((b == 1 or n == 1) and T <= NATIVE_MAX_TOKENS and n < UP_PROJECTED_MIN_TOKENS
+            and (h, nope, r, vd, lora) == (16, 128, 64, 128, 512) and x.is_cuda
+            and cache.rows.device == x.device and cache.dtype == torch.bfloat16
+            and is_tiled(W.q_kva, (h * 192 + 576, H), x.device)
+            and is_tiled(A.uk_tiled, (h, lora, nope), x.device)
+            and is_tiled(A.uv_tiled, (h, vd, lora), x.device)
+            and is_tiled(W.o, (H, h * vd), x.device)):
+        return _decode_step_native(x.contiguous(), W, cache, cos.contiguous(), sin.contiguous(),
+                                   A, eps)
     x2 = x.reshape(T, H)
-    nq = h * (nope + r)
-    # up to 4 tokens: every projection on the vector-ALU row kernel, which
-    # spreads a one-token projection over N/8 lane groups
-    few = (T <= ROWS_MAX_TOKENS and W.q_kva is not None and W.q_kva.dim() == 4 and
-           W.o.dim() == 4 and A.uk_tiled is not None)
-    if (b == 1 or n == 1) and W.q_kva is not None and W.q_kva.dim() == 4 and T <= 64:
-        # q_proj and kv_a_proj in one launch, kv_a's rows straight into the slots
-        q = torch.empty((T, nq), dtype=torch.bfloat16, device=x.device)
-        dst = rows[0] if b == 1 else rows[:, 0]
-        if few:
-            ops.linear_rows(x2, W.q_kva, out=q, out1=dst, n_split=nq)
-        else:
-            ops.linear_split(x2, W.q_kva, q, dst)
-        q = q.view(T, h, nope + r)                         # [T, h, 192]
+    q = ops.linear(x, W.q).view(T, h, nope + r)
+    if b == 1 or n == 1:                               # one row stride: project in place
+        ops.linear(x2, W.kva, out=rows[0] if b == 1 else rows[:, 0])
     else:
-        q = ops.linear(x, W.q).view(T, h, nope + r)
-        if b == 1 or n == 1:                               # one row stride: project in place
-            ops.linear(x2, W.kva, out=rows[0] if b == 1 else rows[:, 0])
-        else:
-            rows.copy_(ops.linear(x2, W.kva).view(b, n, lora + r))
+        rows.copy_(ops.linear(x2, W.kva).view(b, n, lora + r))
     L = cache.current_len
     if n >= UP_PROJECTED_MIN_TOKENS:
         o = _attend_up_projected(q.view(b, n, h, nope + r), cache, W, cos, sin, eps)
         return ops.linear(o, W.o)
     latent, k_pe = cache.get(L)
     small = T <= 64 and A.uk_tiled is not None
-    if few:
-        q_abs = ops.linear_rows(q[..., :nope].transpose(0, 1), A.uk_tiled)     # [h, T, lora]
-    elif small:   # per-head products on strided views, one launch each
+    if small:   # per-head products on strided views, one launch each
         q_abs = ops.linear_batched(q[..., :nope].transpose(0, 1), A.uk_tiled)  # [h, T, lora]
     else:
         q_abs = torch.bmm(q[..., :nope].transpose(0, 1).contiguous(), A.w_uk)
@@ -340,10 +331,32 @@ def _decode_step(x: torch.Tensor, W: MLAWeights, cache: LatentKVCache, rows: tor
     cache._rope_len = L          # the kernel rotated and stored the new keys
     if small:   # o[t, h*v:(h+1)*v] = o_lat[h, t] @ (W_UV[h] * w)^T, written token-major
         o = torch.empty((T, h * vd), dtype=torch.bfloat16, device=x.device)
-        (ops.linear_rows if few else ops.linear_batched)(o_lat, A.uv_tiled,
-                                                         out=o.view(T, h, vd).transpose(0, 1))
+        ops.linear_batched(o_lat, A.uv_tiled, out=o.view(T, h, vd).transpose(0, 1))
     else:
         o = torch.bmm(o_lat, A.w_uv_t).transpose(0, 1).reshape(T, h * vd)
-    if few:
-        return ops.linear_rows(o, W.o).view(b, n, -1)
     return ops.linear(o, W.o).view(b, n, -1)
+
+
+def _decode_step_native(x: torch.Tensor, W: MLAWeights, cache: LatentKVCache, cos: torch.Tensor,
+                        sin: torch.Tensor, A: AbsorbedMLAWeights, eps: float) -> torch.Tensor:
+    """The absorbed step of one sequence, or of one token each, in one C call
+    (dsk_mla_decode_forward): kv_a's output lands in the cache slots, the intermediates
+    in one workspace."""
+    op = "mla_decode_forward"
+    b, n, H = x.shape
+    dev, L = x.device, cache.current_len
+    ops._req(cos.device == dev and sin.device == dev and cos.dtype == torch.bfloat16
+             and sin.dtype == torch.bfloat16, f"{op}: cos and sin must be bf16 CUDA tensors.")
+    out = torch.empty_like(x)
+    if out.numel() == 0:
+        return out
+    ws = torch.empty(lib.dsk_mla_decode_forward_workspace_size(b, n, L), dtype=torch.uint8,
+                     device=dev)
+    with on_device(dev):
+        check(lib.dsk_mla_decode_forward(
+            x.data_ptr(), W.q_kva.data_ptr(), A.uk_tiled.data_ptr(), A.uv_tiled.data_ptr(),
+            W.o.data_ptr(), cache.rows.data_ptr(), cache.rows.stride(1), cache.rows.stride(0),
+            cos.data_ptr(), sin.data_ptr(), eps, W.softmax_scale, b, n, L - n, cache.rope_len, H,
+            out.data_ptr(), ws.data_ptr(), ws.numel(), stream_handle(dev)), op)
+    cache._rope_len = L          # the kernel rotated and stored the new keys
+    return out

@@ -25,7 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from ._lib import check, lib, stream_handle
+from ._lib import check, lib, on_device, stream_handle
 from .expert_prepack import prepack_experts, prepack_with_shared, tile_weights
 
 
@@ -97,7 +97,7 @@ def moe_fused_forward_logits(logits: torch.Tensor, hidden_states: torch.Tensor,
     ws = workspace if workspace is not None and workspace.numel() >= nws else \
         torch.empty(nws, dtype=torch.uint8, device=dev)
     idx, w, offs = _routing_outputs(return_routing, T, top_k, E, dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_fused_forward(
             logits.data_ptr(), hidden_states.data_ptr(), w1.data_ptr(), w2.data_ptr(),
             out.data_ptr(), T, E, top_k, n_shared_groups, H, I, 1 if tiled else 0,
@@ -150,7 +150,7 @@ def moe_layer_forward(hidden_states: torch.Tensor, gate_weight: torch.Tensor,
         torch.empty(nws, dtype=torch.uint8, device=dev)
     idx, w, offs = _routing_outputs(return_routing, T, top_k, E, dev)
     bias = gate_bias.contiguous() if gate_bias is not None else None
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_layer_forward(
             hidden_states.data_ptr(), gate_weight.data_ptr(), _ptr(bias), w1.data_ptr(),
             w2.data_ptr(), out.data_ptr(), T, E, top_k, n_shared_groups, H, I,

@@ -13,7 +13,7 @@ from typing import List
 
 import torch
 
-from ._lib import check, lib, stream_handle
+from ._lib import check, lib, on_device, stream_handle
 
 MAX_EXPERTS = 64
 MAX_TOP_K = 6
@@ -67,7 +67,7 @@ def moe_gate(x: torch.Tensor, weight: torch.Tensor,
         _req(tuple(bias.shape) == (E,), f"{op}: bias must be [{E}].")
     dev = x.device
     logits = torch.empty((T, E), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_gate_logits(x.data_ptr(), x.stride(0), weight.data_ptr(),
                                       bias.data_ptr() if bias is not None else None,
                                       logits.data_ptr(), E, T, E, H, 1 if tiled else 0,
@@ -96,7 +96,7 @@ def moe_routing(logits: torch.Tensor, top_k: int = 6) -> List[torch.Tensor]:
     counts = torch.empty((E,), dtype=torch.int32, device=dev)
     nws = lib.dsk_moe_routing_workspace_size(T, E)
     ws = _ws(nws, dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_routing(logits.data_ptr(), E, idx.data_ptr(), w.data_ptr(),
                                   counts.data_ptr(), T, E, top_k, ws.data_ptr(), ws.numel(),
                                   stream_handle(dev)), op)
@@ -113,7 +113,7 @@ def moe_scan(expert_counts: torch.Tensor) -> torch.Tensor:
     _req(1 <= E <= MAX_EXPERTS, f"{op}: num_experts must be in [1, 64].")
     dev = expert_counts.device
     offsets = torch.empty((E + 1,), dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_scan(expert_counts.data_ptr(), offsets.data_ptr(), E,
                                stream_handle(dev)), op)
     return offsets
@@ -151,7 +151,7 @@ def moe_dispatch(input: torch.Tensor, topk_indices: torch.Tensor, topk_weights: 
     token_map = torch.empty((S,), dtype=torch.int32, device=dev)
     dw = torch.empty((S,), dtype=torch.float32, device=dev)
     ws = _ws(lib.dsk_moe_dispatch_workspace_size(T, E, K), dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_dispatch(input.data_ptr(), H, topk_indices.data_ptr(),
                                    topk_weights.data_ptr(), expert_offsets.data_ptr(),
                                    dispatched.data_ptr(), token_map.data_ptr(), dw.data_ptr(),
@@ -182,7 +182,7 @@ def moe_combine(expert_output: torch.Tensor, token_map: torch.Tensor,
     dev = expert_output.device
     out = torch.empty((int(num_tokens), H), dtype=torch.bfloat16, device=dev)
     ws = _ws(lib.dsk_moe_combine_workspace_size(S, int(num_tokens)), dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_moe_combine(expert_output.data_ptr(), token_map.data_ptr(),
                                   dispatched_weights.data_ptr(), out.data_ptr(), S,
                                   int(num_tokens), H, ws.data_ptr(), ws.numel(),
@@ -201,7 +201,7 @@ def swiglu(input: torch.Tensor) -> torch.Tensor:
     rows, n2 = input.shape
     I = n2 // 2
     out = torch.empty((rows, I), dtype=torch.bfloat16, device=input.device)
-    with torch.cuda.device(input.device):
+    with on_device(input.device):
         check(lib.dsk_swiglu(input.data_ptr(), out.data_ptr(), rows, I,
                              stream_handle(input.device)), op)
     return out
@@ -234,7 +234,7 @@ def moe_gemm1(dispatched: torch.Tensor, packed_w1: torch.Tensor,
     out = torch.empty((S, N), dtype=torch.bfloat16, device=dispatched.device)
     if S == 0:
         return out
-    with torch.cuda.device(dispatched.device):
+    with on_device(dispatched.device):
         check(lib.dsk_moe_gemm1(dispatched.data_ptr(), packed_w1.data_ptr(), out.data_ptr(),
                                 expert_offsets.data_ptr(), S, E, H, N,
                                 stream_handle(dispatched.device)), op)
@@ -254,7 +254,7 @@ def moe_gemm1_swiglu(dispatched: torch.Tensor, packed_w1: torch.Tensor,
     out = torch.empty((S, I), dtype=torch.bfloat16, device=dispatched.device)
     if S == 0:
         return out
-    with torch.cuda.device(dispatched.device):
+    with on_device(dispatched.device):
         check(lib.dsk_moe_gemm1_swiglu(dispatched.data_ptr(), packed_w1.data_ptr(),
                                        out.data_ptr(), expert_offsets.data_ptr(), S, E, H, I,
                                        stream_handle(dispatched.device)), op)
@@ -271,7 +271,7 @@ def moe_gemm2(swiglu_out: torch.Tensor, w2: torch.Tensor,
     out = torch.empty((S, H), dtype=torch.bfloat16, device=swiglu_out.device)
     if S == 0:
         return out
-    with torch.cuda.device(swiglu_out.device):
+    with on_device(swiglu_out.device):
         check(lib.dsk_moe_gemm2(swiglu_out.data_ptr(), w2.data_ptr(), out.data_ptr(),
                                 expert_offsets.data_ptr(), S, E, I, H,
                                 stream_handle(swiglu_out.device)), op)
@@ -310,7 +310,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor = None) -> t
     else:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     if M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_ex(x2.data_ptr(), x2.stride(0), weight.data_ptr(),
                                     1 if tiled else 0, out.data_ptr(), out.stride(0), M, K, N,
                                     stream_handle(x.device)), op)
@@ -340,7 +340,7 @@ def linear_rowsq(x: torch.Tensor, weight: torch.Tensor, col_begin: int, col_end:
          f"{op}: the column range must be 256-aligned inside [0, {N}).")
     ss = torch.empty(((col_end - col_begin) // 256, M), dtype=torch.float32, device=x.device)
     if M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_rowsq(x2.data_ptr(), x2.stride(0), weight.data_ptr(),
                                        out.data_ptr(), N, M, K, N, ss.data_ptr(), M, col_begin,
                                        col_end, stream_handle(x.device)), op)
@@ -360,7 +360,7 @@ def linear_rowscale(x: torch.Tensor, weight: torch.Tensor, row_sumsq: torch.Tens
          f"{op}: row_sumsq must be a contiguous float32 [parts, {M}] CUDA tensor.")
     out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     if M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_rowscale(x2.data_ptr(), x2.stride(0), weight.data_ptr(),
                                           out.data_ptr(), N, M, K, N, row_sumsq.data_ptr(), M,
                                           row_sumsq.shape[0], int(n_cols), float(eps),
@@ -389,7 +389,7 @@ def linear_split(x: torch.Tensor, weight: torch.Tensor, out0: torch.Tensor,
     n0 = out0.shape[1]
     _req(n0 + out1.shape[1] == N, f"{op}: out0 and out1 widths must add up to {N}.")
     if M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_split(x.data_ptr(), x.stride(0), weight.data_ptr(),
                                        out0.data_ptr(), out0.stride(0), out1.data_ptr(),
                                        out1.stride(0), M, K, N, n0, stream_handle(x.device)), op)
@@ -414,7 +414,7 @@ def linear_batched(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor = No
     _req(out.is_cuda and out.dtype == torch.bfloat16 and tuple(out.shape) == (nb, M, N) and
          out.stride(2) == 1, f"{op}: out must be bf16 [{nb}, {M}, {N}] with a contiguous last dim.")
     if nb and M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_batched(x.data_ptr(), x.stride(1), x.stride(0), weight.data_ptr(),
                                          out.data_ptr(), out.stride(1), out.stride(0), nb, M, K,
                                          N, stream_handle(x.device)), op)
@@ -453,7 +453,7 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor = None,
     o0 = out if batched else out[None]
     o1 = (out1 if batched else out1[None]) if out1 is not None else None
     if nb and M:
-        with torch.cuda.device(x.device):
+        with on_device(x.device):
             check(lib.dsk_linear_rows(xb.data_ptr(), xb.stride(1), xb.stride(0), wb.data_ptr(),
                                       wb[0].numel() if wb.shape[0] > 1 else 0, o0.data_ptr(),
                                       o0.stride(1),
@@ -489,7 +489,7 @@ def kv_upproj(normed_kv: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     rows = normed_kv.numel() // r
     out = torch.empty((*normed_kv.shape[:-1], n), dtype=torch.bfloat16, device=normed_kv.device)
     if rows:
-        with torch.cuda.device(normed_kv.device):
+        with on_device(normed_kv.device):
             if tiled:
                 check(lib.dsk_linear_ex(normed_kv.data_ptr(), r, weight.data_ptr(), 1,
                                         out.data_ptr(), n, rows, r, n,
@@ -530,7 +530,7 @@ def rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> to
     if rows == 0:
         return out
     fn = lib.dsk_rms_norm if input.dtype == torch.bfloat16 else lib.dsk_rms_norm_f32
-    with torch.cuda.device(input.device):
+    with on_device(input.device):
         check(fn(x2.data_ptr(), x2.stride(0), weight.data_ptr(), out.data_ptr(), H, rows, H,
                  float(eps), stream_handle(input.device)), op)
     return out
@@ -587,14 +587,14 @@ def attn_softmax_(scores: torch.Tensor, scale: float, causal: bool = True,
         return scores
     st = stream_handle(scores.device)
     if mask is None:
-        with torch.cuda.device(scores.device):
+        with on_device(scores.device):
             check(lib.dsk_attn_softmax(flat.data_ptr(), L, rows, kv_len, q_len, float(scale),
                                        1 if causal else 0, st), op)
         return scores
     _req(scores.dim() == 4, f"{op}: a mask needs 4-D scores [b, h, q_len, L].")
     b, h = scores.shape[0], scores.shape[1]
     m = _expand_mask(op, mask, scores.device, b, h, q_len, kv_len)
-    with torch.cuda.device(scores.device):
+    with on_device(scores.device):
         check(lib.dsk_attn_softmax_masked(
             flat.data_ptr(), L, rows, kv_len, q_len, h, float(scale), 1 if causal else 0,
             m.data_ptr(), 1 if m.dtype == torch.float32 else 0, m.stride(0), m.stride(1),
@@ -639,7 +639,7 @@ def mla_attn_pack(q: torch.Tensor, kv: torch.Tensor, k_pe: torch.Tensor, cos: to
     q_out = torch.empty((b, heads, s, 192), dtype=torch.bfloat16, device=dev)
     k_t = torch.empty((b, heads, 192, sp), dtype=torch.bfloat16, device=dev)
     v = torch.empty((b, heads, sp, 128), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_mla_attn_pack_ex(q.data_ptr(), q.stride(1), kv.data_ptr(), kv.stride(1),
                                        k_pe.data_ptr(), k_pe.stride(1), cb.data_ptr(),
                                        sb.data_ptr(), cb.stride(-2),
@@ -686,7 +686,7 @@ def mla_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Tenso
     out = torch.empty((b, n, heads * 128), dtype=torch.bfloat16, device=dev)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.dsk_mla_prefill_attention(
             q.data_ptr(), q.stride(1), kv.data_ptr(), kv.stride(1), k_rope.data_ptr(),
             k_rope.stride(1), k_rope.stride(0), cb.data_ptr(), sb.data_ptr(), cb.stride(-2),
@@ -782,7 +782,7 @@ def mla_decode_attention(q_abs: torch.Tensor, q_pe: torch.Tensor, latent: torch.
         return out
     ws = _ws(lib.dsk_mla_decode_workspace_size(b, n, L), q_abs.device)
     ld_batch = latent.stride(0) if b > 1 else L * latent.stride(1)
-    with torch.cuda.device(q_abs.device):
+    with on_device(q_abs.device):
         check(lib.dsk_mla_decode_attention(
             q_abs.data_ptr(), q_abs.stride(0), q_abs.stride(1), q_pe.data_ptr(), q_pe.stride(0),
             q_pe.stride(1), latent.data_ptr(), k_pe.data_ptr(), k_rope.data_ptr(), rope_len,
@@ -806,7 +806,7 @@ def rope_single(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
         cos, sin = cos.contiguous(), sin.contiguous()
     sb, sh, ss = _rope_strides(x, "x")
     out = torch.empty((b, h, s, d), dtype=torch.bfloat16, device=x.device)
-    with torch.cuda.device(x.device):
+    with on_device(x.device):
         check(lib.dsk_rope(x.data_ptr(), sb, sh, ss, cos.data_ptr(), sin.data_ptr(), cos.stride(0),
                            cos.stride(2), out.data_ptr(), b, h, s, d,
                            stream_handle(x.device)), op)
@@ -843,7 +843,7 @@ def rope(q_pe: torch.Tensor, k_pe: torch.Tensor, cos: torch.Tensor,
     hk = k_pe.shape[1]
     q_rot = torch.empty((b, hq, s, d), dtype=torch.bfloat16, device=q_pe.device)
     k_rot = torch.empty((b, hk, s, d), dtype=torch.bfloat16, device=q_pe.device)
-    with torch.cuda.device(q_pe.device):
+    with on_device(q_pe.device):
         check(lib.dsk_rope_qk(q_pe.data_ptr(), qsb, qsh, qss, k_pe.data_ptr(), ksb, ksh, kss,
                               cos.data_ptr(), sin.data_ptr(), cb, cs, q_rot.data_ptr(),
                               k_rot.data_ptr(), b, hq, hk, s, d,

@@ -243,6 +243,37 @@ int dsk_mla_prefill_attention(const dsk_bf16* q, int64_t ld_q, const dsk_bf16* k
                               int64_t ld_out, int batch, int q_len, int kv_len, int heads,
                               void* stream);
 
+/* ------------------------------------------------------------- MLA module --
+ * DeepSeekMLA.forward (mla.py:295-393) and a decode step against the latent cache as
+ * one call each: the kernels above on the caller's stream, every intermediate in the
+ * caller's workspace. Head dims 128 + 64 / 128, latent 512; weights fragment-tiled.
+ *   dsk_mla_forward: x bf16 [batch * seq, hidden] contiguous, w_q_kva [heads*192 + 576,
+ *     hidden] (q rows, then kv_a rows), w_kvb [heads*256, 512] with the latent norm
+ *     weight folded into its input columns, w_o [hidden, heads*128]; cos/sin, causal,
+ *     mask and scale as in dsk_mla_prefill_attention; out [batch * seq, hidden].
+ *     heads % 4 == 0.
+ *   dsk_mla_decode_forward: n new tokens of each of `batch` sequences (batch == 1 or
+ *     n == 1, at most 64 tokens), 16 heads. cache_rows: bf16 token rows of 640 values
+ *     (raw latent 512, raw RoPE key 64, rotated key 64) at b * ld_batch + j * ld_tok,
+ *     the first `cached` of them filled, the next n written here; rotated keys below
+ *     rope_len are valid, the others are made. w_uk [16][512, 128], w_uv [16][128, 512]:
+ *     the absorbed per-head up-projections; cos/sin: contiguous [positions, 64]. */
+size_t dsk_mla_forward_workspace_size(int batch, int seq, int heads);
+int dsk_mla_forward(const dsk_bf16* x, const dsk_bf16* w_q_kva, const dsk_bf16* w_kvb,
+                    const dsk_bf16* w_o, const dsk_bf16* cos_t, const dsk_bf16* sin_t,
+                    int64_t ld_cs, int64_t cs_batch_stride, float eps, float scale,
+                    int causal, const void* mask, int mask_dtype, int64_t mask_sb,
+                    int64_t mask_sh, int64_t mask_sq, dsk_bf16* out, int batch, int seq,
+                    int heads, int hidden, void* workspace, size_t workspace_bytes,
+                    void* stream);
+size_t dsk_mla_decode_forward_workspace_size(int batch, int n, int kv_len);
+int dsk_mla_decode_forward(const dsk_bf16* x, const dsk_bf16* w_q_kva, const dsk_bf16* w_uk,
+                           const dsk_bf16* w_uv, const dsk_bf16* w_o, dsk_bf16* cache_rows,
+                           int64_t ld_tok, int64_t ld_batch, const dsk_bf16* cos_t,
+                           const dsk_bf16* sin_t, float eps, float scale, int batch, int n,
+                           int cached, int rope_len, int hidden, dsk_bf16* out,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
 /* --------------------------------------------------------------- rms_norm --
  * y = w * x * rsqrt(mean(x^2) + eps), fp32 math, one rounding of the output.
  * bf16 in/out with fp32 weight: replaces launch_rms_norm

@@ -402,3 +402,43 @@ def test_linear_row_statistics_validation(dsk):
     assert rowscale(parts=3) == 1 and "parts" in _err(dsk)
     assert rowscale(cols=0) == 1 and "cols" in _err(dsk)
     assert rowscale(k=64) == 1 and "K % 128" in _err(dsk)
+
+
+def test_mla_module_validation(dsk):
+    lib = dsk.lib
+
+    def fwd(heads=16, seq=8, ws=256, nbytes=1 << 30, hidden=2048):
+        return lib.dsk_mla_forward(16, 16, 16, 16, 16, 16, 64, 0, 1e-6, 0.1, 1, None, 0, 0, 0, 0,
+                                   16, 1, seq, heads, hidden, ws, nbytes, None)
+    assert fwd(seq=0) == 0
+    assert fwd(heads=6) == 1 and "multiple of 4" in _err(dsk)
+    assert fwd(hidden=0) == 1
+    need = lib.dsk_mla_forward_workspace_size(1, 8, 16)
+    assert fwd(nbytes=need - 1) == 5 and "workspace" in _err(dsk)
+    assert fwd(ws=None) == 5
+
+    def dec(batch=1, n=1, ws=256, nbytes=1 << 30, rows=16, ld_tok=640):
+        return lib.dsk_mla_decode_forward(16, 16, 16, 16, 16, rows, ld_tok, 640 * 100, 16, 16,
+                                          1e-6, 0.1, batch, n, 10, 10, 2048, 16, ws, nbytes, None)
+    assert dec(batch=0) == 0 and dec(n=0) == 0
+    assert dec(batch=2, n=2) == 1 and dec(n=65) == 1 and "at most 64" in _err(dsk)
+    assert dec(ld_tok=576) == 1 and dec(rows=None) == 1
+    need = lib.dsk_mla_decode_forward_workspace_size(1, 1, 11)
+    assert dec(nbytes=need - 1) == 5 and "workspace" in _err(dsk)
+
+
+def test_prefill_attention_validation(dsk):
+    lib = dsk.lib
+
+    def call(q=16, ld_q=3072, ld_kv=4096, ld_kr=64, scale=0.1, mask=None, mkind=0, n=4, L=8,
+             batch=1, out=16, ld_out=2048):
+        return lib.dsk_mla_prefill_attention(q, ld_q, 16, ld_kv, 16, ld_kr, 0, 16, 16, 64, 0,
+                                             scale, 1, mask, mkind, 0, 0, 0, out, ld_out, batch,
+                                             n, L, 16, None)
+    assert call(batch=0) == 0 and call(n=0) == 0
+    assert call(n=9) == 1 and "q_len <= kv_len" in _err(dsk)
+    assert call(scale=0.0) == 1 and call(scale=-1.0) == 1
+    assert call(mask=16, mkind=5) == 1 and "mask dtype" in _err(dsk)
+    assert call(q=None) == 2
+    assert call(q=8) == 3 and call(ld_q=3076) == 3 and call(ld_out=2052) == 3
+    assert call(ld_q=3064) == 1 and call(ld_kv=4088) == 1 and call(ld_kr=56) == 1
