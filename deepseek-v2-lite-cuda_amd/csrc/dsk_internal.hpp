@@ -27,6 +27,8 @@ struct GemmArgs {
   int chunk_m_tiles;       // large-group kernels: M tiles of a typical group, so that
                            // tiles are dealt to the XCDs a group at a time (0: chunks of
                            // up to kTileChunk tiles; gemm_sched.hpp)
+  int zero_uncovered;      // medium-problem kernel, row-major weights: also zero the rows
+                           // outside [offsets[0], offsets[G]) that no group covers
   int chunk;               // tiles per chunk of the deal (set by the launchers)
   int64_t a_group_stride;  // skinny kernel: elements between the A bases of consecutive
   int64_t c_group_stride;  // groups, and of the C bases (0: one base, rows by offsets)

@@ -1528,12 +1528,18 @@ int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
   return g ? run_gemm_t<false, true, false>(a, st) : run_gemm_t<false, false, false>(a, st);
 }
 
-int zero_uncovered_rows(uint16_t* C, int64_t ldc, int M, int N, const int32_t* offsets,
-                        int G, hipStream_t st) {
-  if (M == 0) return DSK_OK;
-  hipLaunchKernelGGL(zero_uncovered_rows_kernel, dim3(64), dim3(256), 0, st, C, ldc, M, N,
-                     offsets, G);
-  return check_launch("zero_uncovered_rows_kernel");
+// A grouped GEMM op on a caller's offsets: rows that no group covers come out zero, in
+// the GEMM's own launch where the kernel does it (a launch of its own took 4 us).
+static int run_op_gemm(GemmArgs a, bool swiglu, hipStream_t st) {
+  if (a.M > kSkinnyMaxRows && mid_gemm_takes(a, swiglu)) {
+    a.zero_uncovered = 1;
+  } else {
+    hipLaunchKernelGGL(zero_uncovered_rows_kernel, dim3(64), dim3(256), 0, st, a.C, a.ldc, a.M,
+                       a.N, a.offsets, a.G);
+    const int rc = check_launch("zero_uncovered_rows_kernel");
+    if (rc) return rc;
+  }
+  return run_gemm(a, swiglu, st);
 }
 
 }  // namespace dsk
@@ -1555,9 +1561,7 @@ extern "C" int dsk_moe_gemm1(const dsk_bf16* dispatched, const dsk_bf16* packed_
   int rc = validate_gemm(a, "moe_gemm1");
   if (rc) return rc;
   hipStream_t st = as_stream(stream);
-  if ((rc = zero_uncovered_rows(out, n_out, total_slots, n_out, expert_offsets, num_experts, st)))
-    return rc;
-  return run_gemm(a, false, st);
+  return run_op_gemm(a, false, st);
 }
 
 extern "C" int dsk_moe_gemm1_swiglu(const dsk_bf16* dispatched, const dsk_bf16* packed_w1,
@@ -1578,10 +1582,7 @@ extern "C" int dsk_moe_gemm1_swiglu(const dsk_bf16* dispatched, const dsk_bf16* 
   int rc = validate_gemm(a, "moe_gemm1_swiglu");
   if (rc) return rc;
   hipStream_t st = as_stream(stream);
-  if ((rc = zero_uncovered_rows(out, intermediate, total_slots, intermediate, expert_offsets,
-                                num_experts, st)))
-    return rc;
-  return run_gemm(a, true, st);
+  return run_op_gemm(a, true, st);
 }
 
 extern "C" int dsk_moe_gemm2(const dsk_bf16* swiglu_out, const dsk_bf16* w2, dsk_bf16* out,
@@ -1599,10 +1600,7 @@ extern "C" int dsk_moe_gemm2(const dsk_bf16* swiglu_out, const dsk_bf16* w2, dsk
   int rc = validate_gemm(a, "moe_gemm2");
   if (rc) return rc;
   hipStream_t st = as_stream(stream);
-  if ((rc = zero_uncovered_rows(out, hidden, total_slots, hidden, expert_offsets, num_experts,
-                                st)))
-    return rc;
-  return run_gemm(a, false, st);
+  return run_op_gemm(a, false, st);
 }
 
 extern "C" int dsk_linear(const dsk_bf16* x, int64_t ld_x, const dsk_bf16* w, dsk_bf16* out,

@@ -89,3 +89,47 @@ def test_fused_layer_groups(dsk, T, bias):
     assert float(err) <= 2.0 ** -7, float(err)
     assert torch.equal(out, dsk.moe_fused_forward_logits(
         logits, x, dsk.tile_weights(w1), dsk.tile_weights(w2), K, nsh, E))
+
+
+@pytest.mark.parametrize("counts", [[65], [64, 0, 1, 33, 31], [40] * 8, [127, 128, 129, 0, 65],
+                                    [300, 2, 0, 70], [500, 20, 20, 20]])
+@pytest.mark.parametrize("I,K", [(96, 64), (192, 192)])
+def test_row_major_groups(dsk, counts, I, K):
+    """The ops on row-major weights: 64- and 128-row tiles, SwiGLU from the halves of a block,
+    uncovered rows zero (3 before the first group, 2 after the last)."""
+    E, S = len(counts), sum(counts) + 5
+    g = torch.Generator().manual_seed(S + I)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(torch.bfloat16).to(DEV)  # noqa: E731
+    x, w1, w2 = rnd(S, K), rnd(E, 2 * I, K), rnd(E, K, I)
+    off = torch.tensor(np.concatenate([[3], 3 + np.cumsum(counts)]), dtype=torch.int32, device=DEV)
+    torch.full((S, 2 * I), float("nan"), dtype=torch.bfloat16, device=DEV)   # stale memory
+    gu = dsk.moe_gemm1(x, w1, off)
+    h = dsk.moe_gemm1_swiglu(x, w1, off)
+    y = dsk.moe_gemm2(h, w2, off) if I % 64 == 0 else None
+    ends = off.cpu().tolist()
+    for e in range(E):
+        r = slice(ends[e], ends[e + 1])
+        if ends[e] == ends[e + 1]:
+            continue
+        _check(gu[r], x[r], w1[e])
+        if y is not None:
+            _check(y[r], h[r], w2[e])
+        a = x[r].double() @ w1[e].double().t()
+        ref = torch.nn.functional.silu(a[:, :I]) * a[:, I:]
+        assert float((h[r].double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    for t in (gu, h) + (() if y is None else (y,)):
+        assert bool((t[:3] == 0).all() and (t[S - 2:] == 0).all())
+
+
+def test_row_major_overlapping_offsets(dsk):
+    """Offsets that decrease: a group's rows are [off[g], max(off[g], off[g + 1])), a row of
+    two groups may come from either, and rows outside [off[0], off[G]) that some group
+    covers are not zeroed."""
+    off = torch.tensor([5, 130, 90, 300, 290], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(320, 128, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(4, 64, 128, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    out = dsk.moe_gemm1(x, w, off)
+    _check(out[5:90], x[5:90], w[0])
+    _check(out[130:300], x[130:300], w[2])
+    assert bool((out[:5] == 0).all() and (out[300:] == 0).all())
