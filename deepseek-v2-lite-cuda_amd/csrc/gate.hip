@@ -10,10 +10,13 @@
 // weight and the torch GEMM launch, which at decode sizes cost more than the
 // dot products.
 //
-// One workgroup per 32 tokens x 32 experts, 16 waves splitting K sixteen ways
-// (a decode step has one or two workgroups, so the K split is what spreads
-// the loads); each wave issues all loads of a chunk of 8 K steps before its
-// MFMAs. The partial sums meet in LDS in a fixed order (waves 1..15 into
+// One workgroup per B tokens x B experts (B = 32, or 16 of the MFMA's 32 rows with
+// the others repeating them), 16 waves splitting K sixteen ways; each wave issues all
+// loads of a chunk of 8 K steps before its MFMAs. A workgroup pulls 2 B rows of x and
+// weights through one CU, which holds ~64 lines in flight, so that stream is its time:
+// blocks of 16 halve it and spread the work over four times the CUs (T = 32 and 600:
+// 16.1 us with blocks of 32, 11.1 and 11.6 with 16); from 2048 tokens up the blocks of 32
+// cover the CUs and read x half as often. The partial sums meet in LDS in a fixed order (waves 1..15 into
 // wave 0), so the result is the same on every run.
 #include "dsk_internal.hpp"
 #include "gate_parts.hpp"
@@ -22,16 +25,18 @@ namespace dsk {
 
 constexpr int kGateWaves = 16;
 
-template <bool TILED>
+template <bool TILED, int B>
 __global__ __launch_bounds__(64 * kGateWaves) void gate_logits_kernel(
     const uint16_t* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ wg,
     const float* __restrict__ bias, float* __restrict__ logits, int64_t ld_out, int T, int E,
     int H) {
-  __shared__ floatx4_t red[kGateWaves - 1][4][64];
+  static_assert(B == 16 || B == 32, "block of 16 or 32");
+  constexpr int QG = B / 8;  // groups of 8 expert rows that hold results
+  __shared__ floatx4_t red[kGateWaves - 1][QG][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int t0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
-  const int r32 = lane & 31, h = lane >> 5;
+  const int t0 = blockIdx.x * B, e0 = blockIdx.y * B;
+  const int r32 = lane & (B - 1), h = lane >> 5;
   // weights are MFMA operand A (output rows = experts), tokens operand B
   const int e = min(e0 + r32, E - 1);
   const int t = min(t0 + r32, T - 1);
@@ -39,8 +44,9 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_logits_kernel(
   // row-major weight: row e, 16 elements per K step (each load touches 32
   // rows); fragment-tiled weight: fragment (expert block, K step) is 512
   // consecutive elements, lane-ordered (each load reads 1 KB contiguous)
-  const uint16_t* wrow = TILED ? wg + ((int64_t)blockIdx.y * ksteps) * 512 + lane * 8
-                               : wg + (int64_t)e * H + 8 * h;
+  const uint16_t* wrow =
+      TILED ? wg + ((int64_t)(e0 / 32) * ksteps) * 512 + ((e0 & 31) + r32 + 32 * h) * 8
+            : wg + (int64_t)e * H + 8 * h;
   constexpr int kWStep = TILED ? 512 : 16;
   const uint16_t* xrow = x + (int64_t)t * ld_x + 8 * h;
   const int s_beg = wave * ksteps / kGateWaves;
@@ -67,7 +73,7 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_logits_kernel(
 
   if (wave > 0) {
 #pragma unroll
-    for (int qg = 0; qg < 4; ++qg) {
+    for (int qg = 0; qg < QG; ++qg) {
       floatx4_t v;
 #pragma unroll
       for (int c = 0; c < 4; ++c) v[c] = acc[4 * qg + c];
@@ -77,10 +83,10 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_logits_kernel(
   __syncthreads();
   if (wave != 0) return;
   const int tok = t0 + r32;
-  if (tok >= T) return;
+  if ((lane & 31) >= B || tok >= T) return;
   float* orow = logits + (int64_t)tok * ld_out;
 #pragma unroll
-  for (int qg = 0; qg < 4; ++qg) {
+  for (int qg = 0; qg < QG; ++qg) {
     floatx4_t v;
 #pragma unroll
     for (int c = 0; c < 4; ++c) v[c] = acc[4 * qg + c];
@@ -121,8 +127,10 @@ int gate_parts_count(int T, int E, int H) {
 int launch_gate_logits(const uint16_t* x, int64_t ld_x, const uint16_t* wg, bool tiled,
                        const float* bias, float* logits, int64_t ld_out, int T, int E, int H,
                        hipStream_t st) {
-  dim3 grid((T + 31) / 32, (E + 31) / 32);
-  auto kern = tiled ? gate_logits_kernel<true> : gate_logits_kernel<false>;
+  const int B = T < 2048 ? 16 : 32;
+  dim3 grid((T + B - 1) / B, (E + B - 1) / B);
+  auto kern = B == 16 ? (tiled ? gate_logits_kernel<true, 16> : gate_logits_kernel<false, 16>)
+                      : (tiled ? gate_logits_kernel<true, 32> : gate_logits_kernel<false, 32>);
   hipLaunchKernelGGL(kern, grid, dim3(64 * kGateWaves), 0, st, x, ld_x, wg, bias, logits, ld_out,
                      T, E, H);
   return check_launch("gate_logits_kernel");

@@ -177,7 +177,11 @@ def route_dispatch_combine(hidden_states: torch.Tensor, gate_weight: torch.Tenso
     """The reference op sequence (moe_fused.py:118-154) over this package's ops:
     routing -> scan -> dispatch -> gemm1 -> swiglu -> gemm2 -> combine."""
     T = hidden_states.shape[0]
-    logits = F.linear(hidden_states.float(), gate_weight.float(), None)
+    if (gate_weight.dim() == 2 and gate_weight.is_contiguous() and gate_weight.shape[1] % 16 == 0
+            and gate_weight.data_ptr() % 16 == 0):
+        logits = gate_logits(hidden_states, gate_weight)
+    else:
+        logits = F.linear(hidden_states.float(), gate_weight.float(), None)
     topk_indices, topk_weights, expert_counts = ops.moe_routing(logits, top_k)
     expert_offsets = ops.moe_scan(expert_counts)
     dispatched, token_map, dispatched_weights = ops.moe_dispatch(

@@ -171,6 +171,45 @@ def test_combine_zero_weights_and_empty_tokens(dsk):
     assert torch.all(out[5:] == 0)
 
 
+@pytest.mark.parametrize("T,S", [(1, 3), (5, 64), (9, 65), (4, 700), (2000, 12000), (6000, 9000), (9000, 9000),
+                                 (7, 0)])
+def test_combine_list_and_route_edges(dsk, T, S):
+    """Slot lists at and past the 64 entries a workgroup holds (4 tokens of 700 slots), the
+    largest maps that are scanned, maps past that, and slots of no token."""
+    g = torch.Generator().manual_seed(T + S)
+    y = torch.randn(S, 64, generator=g).to(torch.bfloat16)
+    tm = torch.randint(-1, T + 1, (S,), generator=g, dtype=torch.int32)
+    _combine_case(dsk, y, tm, torch.rand(S, generator=g) / 8, T)
+
+
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 257, 4096, 4097])
+def test_dispatch_repeats_and_out_of_range_experts(dsk, T):
+    """Stable slots when rows repeat an expert or name none (both skipped), on either side
+    of the token count that one launch takes."""
+    E, K, H = 7, 4, 64
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    idx = torch.randint(-1, E + 2, (T, K), generator=g, dtype=torch.int32)
+    w = torch.rand(T, K, generator=g)
+    slots = [[] for _ in range(E)]
+    for t in range(T):
+        seen = set()
+        for k in range(K):
+            e = int(idx[t, k])
+            if 0 <= e < E and e not in seen:
+                slots[e].append((t, k))
+            seen.add(e)
+    off = np.concatenate([[0], np.cumsum([len(s) for s in slots])]).astype(np.int32)
+    disp, tm, dw = dsk.moe_dispatch(x.to(DEV), idx.to(DEV), w.to(DEV), torch.from_numpy(off).to(DEV))
+    flat = [p for s in slots for p in s]
+    n = len(flat)
+    if n:
+        t, k = (torch.tensor(v) for v in zip(*flat))
+        assert torch.equal(tm[:n].cpu().long(), t)
+        assert torch.equal(dw[:n].cpu(), w[t, k])
+        assert torch.equal(disp[:n].cpu(), x[t])
+
+
 # ------------------------------------------------------------------- swiglu --
 @pytest.mark.parametrize("rows", [0, 1, 8, 256])
 def test_swiglu(dsk, rows):
