@@ -168,6 +168,13 @@ template <int kCtrl>
 __device__ __forceinline__ int dpp_i32(int v) {
   return __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xf, 0xf, false);
 }
+__device__ __forceinline__ uint32_t row16_max(uint32_t v) {
+  v = max(v, (uint32_t)dpp_i32<0xB1>((int)v));
+  v = max(v, (uint32_t)dpp_i32<0x4E>((int)v));
+  v = max(v, (uint32_t)dpp_i32<0x141>((int)v));
+  v = max(v, (uint32_t)dpp_i32<0x140>((int)v));
+  return v;
+}
 __device__ __forceinline__ int row16_min(int v) {
   v = min(v, dpp_i32<0xB1>(v));
   v = min(v, dpp_i32<0x4E>(v));

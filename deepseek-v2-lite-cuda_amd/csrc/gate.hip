@@ -20,6 +20,7 @@
 // wave 0), so the result is the same on every run.
 #include "dsk_internal.hpp"
 #include "gate_parts.hpp"
+#include "route_token.hpp"
 
 namespace dsk {
 
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(64) void gate_parts_kernel(
 int gate_parts_count(int T, int E, int H) {
   const int blocks = ((T + 31) / 32) * ((E + 31) / 32);
   int n = 512 / blocks;
-  n = n < 1 ? 1 : (n > 4 ? 4 : n);
+  n = n < 1 ? 1 : (n > kMaxGateParts ? kMaxGateParts : n);
   return n > H / 16 ? H / 16 : n;
 }
 

@@ -647,6 +647,8 @@ int launch_route(const float* logits, int64_t ld, int n_parts, int64_t part_stri
                  float* w, int32_t* blk_hist, int32_t* local_rank, int32_t* counts,
                  int32_t* offsets, int32_t* token_map, int32_t* slot_of,
                  int n_extra_groups, hipStream_t st) {
+  DSK_REQUIRE(n_parts >= 1 && n_parts <= kMaxGateParts, DSK_ERR_INVALID_ARG,
+              "route: too many planes of partial gate sums");
   // a single chunk (T <= 64) launches only the waves its tokens need (at
   // least one: wave 0 does the chunk's scan; 64 lanes cover the 64 experts)
   const int threads =

@@ -94,6 +94,30 @@ def test_routing_ties_and_determinism(dsk):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("T,E,K", [(1, 64, 6), (61, 64, 6), (130, 40, 5), (67, 5, 5)])
+def test_routing_signed_zeros_infinities_and_nan(dsk, T, E, K):
+    """Picks compared as unsigned keys: the order of the floats, with -0 equal to +0 and
+    NaN as -inf (ties to the lower index), and weights as a float softmax gives them: NaN
+    rows where a logit is NaN or +inf, exact zeros for -inf picks."""
+    g = torch.Generator().manual_seed(T + E)
+    vals = torch.tensor([0.0, -0.0, 1e-40, -1e-40, 3e38, -3e38, float("inf"), float("-inf"),
+                         float("nan"), 1.0, -1.0])
+    logits = torch.randn(T, E, generator=g)
+    special = torch.rand(T, E, generator=g) < 0.3
+    logits[special] = vals[torch.randint(0, len(vals), (T, E), generator=g)][special]
+    logits[0, 1:] = float("-inf")                    # fewer choices than picks
+    logits[T // 2] = torch.where(torch.rand(E, generator=g) < 0.5, 0.0, -0.0)
+    idx, w, counts = dsk.moe_routing(logits.to(DEV), K)
+    order = torch.nan_to_num(logits.double(), nan=float("-inf"), posinf=float("inf"),
+                             neginf=float("-inf"))
+    ref = torch.sort(order, dim=1, descending=True, stable=True).indices[:, :K]
+    assert torch.equal(idx.cpu().long(), ref)
+    assert torch.equal(counts.cpu().long(), torch.bincount(ref.flatten(), minlength=E))
+    rw = torch.softmax(logits.double(), 1).gather(1, ref)
+    # fp32 exp and a sum of at most 64 terms: well inside 64 x 2^-23 of the value
+    torch.testing.assert_close(w.cpu().double(), rw, rtol=F32_TOL, atol=1e-38, equal_nan=True)
+
+
 # --------------------------------------------------------------------- scan --
 @pytest.mark.parametrize("case", GOLD["scan"], ids=lambda c: c["name"])
 def test_scan_kat(dsk, case):
