@@ -76,6 +76,14 @@ struct GemmArgs {
 constexpr int kRouteInGemmTokens = 1;
 constexpr int kRouteInGemmSlots = 256;  // routed + always-on rows the prologue maps
 
+// Tokens up to which the layer's second GEMM and its combine run as one launch (gemv.hip).
+constexpr int kGemm2CombineTokens = 2;
+bool gemm2_combine_takes(int T, int K, int G, int nsh, int H, int I);
+int launch_gemm2_combine(const uint16_t* h, const uint16_t* w2, bool tiled,
+                         const int32_t* offsets, const int32_t* slot_of, const float* topk_w,
+                         uint16_t* out, int T, int K, int G, int nsh, int H, int I,
+                         hipStream_t st);
+
 int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st);
 // The medium-problem kernel (gemm_mid.hip): whether it takes a problem (it is then the
 // faster one), and its launch.

@@ -17,6 +17,8 @@
 // on every run.
 #include "dsk_internal.hpp"
 
+#include <climits>
+
 namespace dsk {
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -121,6 +123,172 @@ __global__ __launch_bounds__(64) void linear_rows_kernel(RowsArgs a) {
                                   : a.out1 + b * a.out1_bs + m * a.ld_out1 + (n - a.n_split);
     *dst = f32_to_bf16(v);
   }
+}
+
+// ------------------------------------------- down projection + combine ----
+// The MoE layer's second GEMM and its combine in one launch, for the smallest steps:
+//
+//   out[t][n] = sum_k wt[t][k] * y[slot_of[t][k]][n] + sum_x y[S + x T + t][n],
+//   y[s][n] = bf16(sum_i h[s][i] * w2[g(s)][n][i])
+//
+// with the rounding of y and the order of the sum (slots ascending, then the always-on
+// groups, fp32, one rounding) of combine_slots_kernel.
+//
+// At one token the GEMM streams 46 MB for 12 us and the combine that follows costs a launch
+// (4.6 us) for 32 KB. Both are one launch if a workgroup has the same columns of every
+// busy group, and the even split of the columns also gives each CU the same bytes: a
+// workgroup owns 8 columns (one 128-byte line of each fragment half, as above), each of its
+// 8 waves takes every eighth busy group, all weight loads of a 1408-long row in flight at
+// once, and the rows of y meet in LDS. The layer at one token 39.0 -> 36.6 us, at two
+// tokens with 9 busy groups 49 -> 44 and with 13 58 -> 58. From three tokens up a wave's
+// bursts over several groups no longer fill the CU's queue (three tokens with 17 to 19 busy
+// groups 76 -> 79 us, four 82 -> 93), so larger steps keep the two launches.
+constexpr int kCombineWavesG2 = 8;
+constexpr int kCombineCols = 8;
+constexpr int kG2Batch = 3;    // 8-element K chunks per lane in flight (1408 = 2.75 x 512)
+constexpr int kG2MaxSlots = 256;
+constexpr int kG2MaxK = 8;
+
+struct Gemm2CombineArgs {
+  const uint16_t* h;  // [slots, I]
+  const uint16_t* w2; // [G, H, I], row-major or tiled
+  const int32_t* offsets;  // [G + 1]
+  const int32_t* slot_of;  // [T, K]
+  const float* topk_w;     // [T, K]
+  uint16_t* out;           // [T, H]
+  int T, K, G, nsh, H, I, slots;
+};
+
+template <int MT, bool TILED>
+__global__ __launch_bounds__(64 * kCombineWavesG2) void gemm2_combine_kernel(Gemm2CombineArgs a) {
+  __shared__ __attribute__((aligned(16))) float s_y[kG2MaxSlots][kCombineCols];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * kCombineCols;
+  const int nch = a.I / 8;
+
+  // busy groups, lane = group (G <= 128: two halves)
+  int lo0 = 0, hi0 = 0, lo1 = 0, hi1 = 0;
+  if (lane < a.G) {
+    lo0 = min(max(a.offsets[lane], 0), a.slots);
+    hi0 = min(max(a.offsets[lane + 1], lo0), a.slots);
+  }
+  if (lane + 64 < a.G) {
+    lo1 = min(max(a.offsets[lane + 64], 0), a.slots);
+    hi1 = min(max(a.offsets[lane + 65], lo1), a.slots);
+  }
+  // the combine's slots and weights of token tid / 8, in ascending slot order, while the
+  // weights stream
+  const int t = tid / kCombineCols, col = tid % kCombineCols;
+  int s[kG2MaxK];
+  float wt[kG2MaxK];
+#pragma unroll
+  for (int k = 0; k < kG2MaxK; ++k) {
+    const bool on = t < a.T && k < a.K;
+    const int sk = on ? a.slot_of[t * a.K + k] : -1;
+    s[k] = sk >= 0 && sk < a.slots ? sk : INT_MAX;
+    wt[k] = on ? a.topk_w[t * a.K + k] : 0.f;
+  }
+  const uint64_t m0 = __ballot(hi0 > lo0), m1 = __ballot(hi1 > lo1);
+  const int c0 = __popcll(m0), busy = c0 + __popcll(m1);
+
+  for (int ord = wave; ord < busy; ord += kCombineWavesG2) {
+    // the ord-th busy group
+    const bool upper = ord >= c0;
+    const uint64_t mask = upper ? m1 : m0;
+    const int want = upper ? ord - c0 : ord;
+    const bool mine = ((mask >> lane) & 1) && __popcll(mask & ((1ull << lane) - 1ull)) == want;
+    const int src = __ffsll((unsigned long long)__ballot(mine)) - 1;
+    const int g = src + (upper ? 64 : 0);
+    const int lo = __builtin_amdgcn_readlane(upper ? lo1 : lo0, src);
+    const int rows = min(__builtin_amdgcn_readlane(upper ? hi1 : hi0, src) - lo, MT);
+    const uint16_t* wb = a.w2 + (int64_t)g * a.H * a.I;
+    wb += TILED ? (int64_t)(n0 / 32) * (a.I / 16) * 512 + (n0 % 32 / kCombineCols) * 64
+                : (int64_t)n0 * a.I;
+    float acc[MT][kCombineCols];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int i = 0; i < kCombineCols; ++i) acc[m][i] = 0.f;
+    for (int j0 = 0; j0 < nch; j0 += 64 * kG2Batch) {
+      u32x4_t wv[kG2Batch][kCombineCols], xv[kG2Batch][MT];
+#pragma unroll
+      for (int u = 0; u < kG2Batch; ++u) {
+        const int c = min(j0 + 64 * u + lane, nch - 1);  // past the row: reload, unused
+        const uint16_t* wp = TILED ? wb + (c >> 1) * 512 + (c & 1) * 256 : wb + c * 8;
+#pragma unroll
+        for (int i = 0; i < kCombineCols; ++i)
+          wv[u][i] = *reinterpret_cast<const u32x4_t*>(wp + (int64_t)i * (TILED ? 8 : a.I));
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          xv[u][m] = *reinterpret_cast<const u32x4_t*>(a.h + (int64_t)(lo + min(m, rows - 1)) * a.I +
+                                                       c * 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // every load of the batch before the first use
+#pragma unroll
+      for (int u = 0; u < kG2Batch; ++u) {
+        if (j0 + 64 * u + lane < nch) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < kCombineCols; ++i)
+              acc[m][i] = dot8(wv[u][i], xv[u][m], acc[m][i]);
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      if (m < rows) {  // uniform
+        float v[kCombineCols];
+#pragma unroll
+        for (int i = 0; i < kCombineCols; ++i) v[i] = bf16_to_f32(f32_to_bf16(wave_sum(acc[m][i])));
+        if (lane == 0) {
+#pragma unroll
+          for (int i = 0; i < kCombineCols; ++i) s_y[lo + m][i] = v[i];
+        }
+      }
+    }
+  }
+  // fixed sorting network on compile-time indices
+#pragma unroll
+  for (int x = 0; x < kG2MaxK; ++x) {
+#pragma unroll
+    for (int y = 0; y < kG2MaxK - 1 - x; ++y) {
+      if (s[y] > s[y + 1]) {
+        const int ts = s[y]; s[y] = s[y + 1]; s[y + 1] = ts;
+        const float tw = wt[y]; wt[y] = wt[y + 1]; wt[y + 1] = tw;
+      }
+    }
+  }
+  __syncthreads();
+  if (t >= a.T) return;
+  float o = 0.f;
+#pragma unroll
+  for (int k = 0; k < kG2MaxK; ++k)
+    if (s[k] != INT_MAX) o = fmaf(wt[k], s_y[s[k]][col], o);
+  for (int x = 0; x < a.nsh; ++x) o += s_y[a.T * a.K + x * a.T + t][col];
+  a.out[(int64_t)t * a.H + n0 + col] = f32_to_bf16(o);
+}
+
+bool gemm2_combine_takes(int T, int K, int G, int nsh, int H, int I) {
+  return T >= 1 && T <= kGemm2CombineTokens && K <= kG2MaxK && G <= 128 &&
+         T * (K + nsh) <= kG2MaxSlots && H % 32 == 0 && I % 16 == 0;
+}
+
+int launch_gemm2_combine(const uint16_t* h, const uint16_t* w2, bool tiled,
+                         const int32_t* offsets, const int32_t* slot_of, const float* topk_w,
+                         uint16_t* out, int T, int K, int G, int nsh, int H, int I,
+                         hipStream_t st) {
+  DSK_REQUIRE(gemm2_combine_takes(T, K, G, nsh, H, I), DSK_ERR_INVALID_ARG,
+              "gemm2_combine: sizes out of range");
+  const Gemm2CombineArgs a{h, w2, offsets, slot_of, topk_w, out, T, K, G, nsh, H, I,
+                           T * (K + nsh)};
+  const dim3 grid((unsigned)(H / kCombineCols));
+  static_assert(kGemm2CombineTokens == 2, "a variant per token count");
+  auto kern = T == 1 ? (tiled ? gemm2_combine_kernel<1, true> : gemm2_combine_kernel<1, false>)
+                     : (tiled ? gemm2_combine_kernel<2, true> : gemm2_combine_kernel<2, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * kCombineWavesG2), 0, st, a);
+  return check_launch("gemm2_combine_kernel");
 }
 
 template <int LPR>

@@ -159,21 +159,28 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
   if ((rc = run_gemm(g1, true, st))) return rc;
   if ((rc = mark(2))) return rc;
 
-  GemmArgs g2{};
-  g2.A = h; g2.lda = I;
-  g2.B = w2; g2.ldb = I; g2.b_group_stride = (int64_t)H * I;
-  g2.C = y; g2.ldc = H;
-  g2.offsets = offsets; g2.G = G;
-  g2.M = Stot; g2.N = H; g2.K = I;
-  g2.offsets_sorted = 1;
-  g2.max_group_rows = T;
-  g2.b_tiled = weight_layout == DSK_LAYOUT_TILED;
-  g2.chunk_m_tiles = g1.chunk_m_tiles;
-  if ((rc = run_gemm(g2, false, st))) return rc;
-  if ((rc = mark(3))) return rc;
+  if (gemm2_combine_takes(T, K, G, nsh, H, I)) {
+    rc = launch_gemm2_combine(h, w2, weight_layout == DSK_LAYOUT_TILED, offsets, slot_of, w, out,
+                              T, K, G, nsh, H, I, st);
+    if (rc) return rc;
+    if ((rc = mark(3))) return rc;
+  } else {
+    GemmArgs g2{};
+    g2.A = h; g2.lda = I;
+    g2.B = w2; g2.ldb = I; g2.b_group_stride = (int64_t)H * I;
+    g2.C = y; g2.ldc = H;
+    g2.offsets = offsets; g2.G = G;
+    g2.M = Stot; g2.N = H; g2.K = I;
+    g2.offsets_sorted = 1;
+    g2.max_group_rows = T;
+    g2.b_tiled = weight_layout == DSK_LAYOUT_TILED;
+    g2.chunk_m_tiles = g1.chunk_m_tiles;
+    if ((rc = run_gemm(g2, false, st))) return rc;
+    if ((rc = mark(3))) return rc;
 
-  rc = launch_combine_slots(y, H, slot_of, w, T, K, H, S, nsh, out, H, st);
-  if (rc) return rc;
+    rc = launch_combine_slots(y, H, slot_of, w, T, K, H, S, nsh, out, H, st);
+    if (rc) return rc;
+  }
   if ((rc = mark(4))) return rc;
   if (expert_offsets_out != nullptr) {
     if (hipMemcpyAsync(expert_offsets_out, offsets, (size_t)(E + 1) * 4,

@@ -649,6 +649,47 @@ def test_fused_layer_small_shapes_routing_and_output(dsk, T, E, K, nsh):
     assert max_rel_err(np32(out), ref) <= BF16_TOL
 
 
+@pytest.mark.parametrize("T,E,K,nsh,H,I", [
+    (1, 64, 6, 2, 2048, 1408), (2, 64, 6, 2, 2048, 1408), (1, 32, 1, 0, 64, 64),
+    (2, 32, 6, 3, 320, 1600), (2, 64, 5, 40, 192, 192), (1, 64, 6, 64, 128, 576)])
+@pytest.mark.parametrize("layout", ["row_major", "tiled"])
+def test_smallest_steps_against_fp64(dsk, T, E, K, nsh, H, I, layout):
+    """The kernels of one- and two-token steps (whole rows per lane group, the down
+    projection and the combine in one launch) at rows shorter than a wave's chunks, rows of
+    more than one batch of chunks, group counts beyond 64 and no always-on groups.
+
+    h, y and the output are each rounded to bf16 once (2^-8 of the value at most; the fp32
+    sums add less than a hundredth of that): |error| <= 2^-8 (sum_s w |W2| |h| + sum_s w |y|
+    + |out|)."""
+    g = torch.Generator().manual_seed(T + E + I)
+    G = E + nsh
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(DEV)
+    w1 = (torch.randn(G, 2 * I, H, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    w2 = (torch.randn(G, H, I, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    wg = (torch.randn(E, H, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    args = (wg, w1, w2) if layout == "row_major" else (
+        dsk.tile_weights(wg[None])[0], dsk.tile_weights(w1), dsk.tile_weights(w2))
+    out, (idx, w, off) = dsk.moe_layer_forward(x, *args, K, nsh, return_routing=True)
+    lg = (x.double() @ wg.double().T).float().cpu().numpy()
+    ridx, rw, rcounts = om.route(lg, K)
+    np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
+    np.testing.assert_array_equal(off.cpu().numpy()[:E + 1], om.scan(rcounts))
+    np.testing.assert_allclose(np32(w), rw, rtol=1e-4)
+    ref = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    room = torch.zeros_like(ref)
+    for t in range(T):
+        picks = [(int(e), float(v)) for e, v in zip(idx[t], w[t])]
+        for e, v in picks + [(E + j, 1.0) for j in range(nsh)]:
+            gu = w1[e].double() @ x[t].double()
+            h = torch.nn.functional.silu(gu[:I]) * gu[I:]
+            y = w2[e].double() @ h
+            ref[t] += v * y
+            room[t] += v * (w2[e].double().abs() @ h.abs() + y.abs())
+    room += ref.abs()
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * 1.01 * room).all())
+    assert torch.equal(out, dsk.moe_layer_forward(x, *args, K, nsh))
+
+
 # -------------------------------------------- module-level drop-in (a10) --
 # A DeepSeekMoE-shaped module (reference moe.py:6-75: gate.weight,
 # experts[i].{gate,up,down}_proj as bias-free nn.Linear, shared_experts,
