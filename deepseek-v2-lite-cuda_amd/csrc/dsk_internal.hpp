@@ -51,31 +51,13 @@ struct GemmArgs {
   int64_t ld_rowscale;
   int rowscale_parts, rowscale_cols;
   float rowscale_eps;
-  // Small-group SwiGLU kernel with gathered rows, optional (decode steps of at
-  // most kRouteInGemmTokens tokens): every workgroup routes the step itself in
-  // its prologue from the gate's partial planes (route_token), and uses its own
-  // expert offsets and row map instead of offsets / a_rows; workgroup 0 also
-  // writes the routing outputs (topk idx / weights, counts, offsets with the
-  // always-on groups, token_map, slot_of) for the kernels after it.
-  const float* rt_parts;
-  int rt_n_parts;
-  int64_t rt_part_stride;
-  const float* rt_bias;
-  int rt_T, rt_E, rt_K, rt_nsh;
-  int32_t* rt_idx;
-  float* rt_w;
-  int32_t* rt_counts;
-  int32_t* rt_offsets;
-  int32_t* rt_token_map;
-  int32_t* rt_slot_of;
 };
 
-// Tokens up to which a decode step is routed in GEMM1's prologue: every launched
-// workgroup routes before it knows whether its group is busy, and at T = 1 the
-// grid holds only busy groups (at most T*K + always-on groups of rows).
-constexpr int kRouteInGemmTokens = 1;
-constexpr int kRouteInGemmSlots = 256;  // routed + always-on rows the prologue maps
-
+// Routing and first GEMM of a one-token layer as one launch (gemv.hip).
+int launch_token_gemm1(const float* parts, int n_parts, int64_t part_stride, const float* bias,
+                       const uint16_t* x, const uint16_t* w1, bool tiled, uint16_t* h, int E,
+                       int K, int nsh, int H, int I, int32_t* idx, float* w, int32_t* counts,
+                       int32_t* offsets, int32_t* token_map, int32_t* slot_of, hipStream_t st);
 // Tokens up to which the layer's second GEMM and its combine run as one launch (gemv.hip).
 constexpr int kGemm2CombineTokens = 2;
 bool gemm2_combine_takes(int T, int K, int G, int nsh, int H, int I);

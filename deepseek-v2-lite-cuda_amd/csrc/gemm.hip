@@ -48,7 +48,6 @@
 #include "dsk_internal.hpp"
 #include "gemm_common.hpp"
 #include "gemm_sched.hpp"
-#include "route_token.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -917,72 +916,6 @@ constexpr int kSkinnyMaxRows = 64;  // largest group the small-group kernel is c
 template <int MT>
 constexpr int skinny_batch() { return MT == 1 ? 4 : 2; }
 
-// Routing of a decode step (at most kRouteInGemmTokens tokens) in the prologue
-// of the small-group SwiGLU kernel, as route_kernel does it for one chunk: the
-// 16-lane row g of wave w picks the experts of token 4 w + g (route_token);
-// 64-bit expert masks in the LDS give each (token, k) its stable slot (expert-
-// major, ascending token) and the offsets of the routed groups, followed by
-// the always-on groups of T rows each. Every workgroup computes the same
-// integers from the same planes; workgroup 0 also stores them for the kernels
-// after this one.
-__device__ __forceinline__ void skinny_route_prologue(const GemmArgs& p,
-                                                      unsigned long long* rt_mask, int* rt_off,
-                                                      int* rt_tok, int lane, int wave,
-                                                      bool store) {
-  const int T = p.rt_T, E = p.rt_E, K = p.rt_K, nsh = p.rt_nsh;
-  if (threadIdx.x < 64) rt_mask[threadIdx.x] = 0ull;
-  __syncthreads();
-  const int j = lane & 15;
-  const int tl = 4 * wave + (lane >> 4);
-  int my_e;
-  float my_w;
-  route_token(p.rt_parts, E, p.rt_n_parts, p.rt_part_stride, p.rt_bias, tl, tl < T,
-              4 * wave < T, E, K, lane, my_e, my_w);
-  if (tl < T && j < K) {
-    atomicOr(&rt_mask[my_e], 1ull << tl);
-    if (store) {
-      p.rt_idx[tl * K + j] = my_e;
-      p.rt_w[tl * K + j] = my_w;
-    }
-  } else {
-    my_e = -1;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    const int c = lane < E ? __popcll(rt_mask[lane]) : 0;
-    const int inc = wave_inclusive_scan(c);
-    if (lane < E) {
-      rt_off[lane] = inc - c;
-      if (store) {
-        p.rt_offsets[lane] = inc - c;
-        p.rt_counts[lane] = c;
-      }
-    }
-    if (lane == 63) {
-      for (int x = 0; x <= nsh; ++x) {
-        rt_off[E + x] = inc + x * T;
-        if (store) p.rt_offsets[E + x] = inc + x * T;
-      }
-    }
-  }
-  __syncthreads();
-  if (my_e >= 0) {
-    const int slot = rt_off[my_e] + __popcll(rt_mask[my_e] & ((1ull << tl) - 1ull));
-    rt_tok[slot] = tl;
-    if (store) {
-      p.rt_token_map[slot] = tl;
-      p.rt_slot_of[tl * K + j] = slot;
-    }
-  }
-  // rows of the always-on groups: group E+x row t is token t
-  const int S = T * K;
-  for (int r = threadIdx.x; r < nsh * T; r += blockDim.x) {
-    rt_tok[S + r] = r % T;
-    if (store) p.rt_token_map[S + r] = r % T;
-  }
-  __syncthreads();
-}
-
 // NB: 32-row weight blocks per workgroup (SwiGLU with NB = 2: a gate and an up
 // block of 32 output columns; SwiGLU with NB = 1: one block whose rows 0-15 are
 // the gate rows and 16-31 the up rows of 16 output columns);
@@ -998,23 +931,9 @@ __device__ __forceinline__ void skinny_gemm_body(const GemmArgs& p, int n_blocks
   static_assert(NW == 4 || NW == 8, "reduction written for 4 or 8 waves");
   // partial sums of the upper half of the waves (8 waves), then of waves 1..3
   __shared__ floatx4_t red[NW == 8 ? 4 : 3][NB][MT][4][64];
-  // routing in the prologue (SwiGLU with gathered rows only): expert masks of
-  // the step's tokens, group offsets and the slot -> token map
-  constexpr bool kCanRoute = SWIGLU && GATHER && NW == 4;
-  __shared__ unsigned long long rt_mask[kCanRoute ? 64 : 1];
-  __shared__ int rt_off[kCanRoute ? kMaxGroups + 1 : 1];
-  __shared__ int rt_tok[kCanRoute ? kRouteInGemmSlots : 1];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  bool routed = false;
-  if constexpr (kCanRoute) {
-    if (p.rt_parts != nullptr) {
-      routed = true;
-      skinny_route_prologue(p, rt_mask, rt_off, rt_tok, lane, wave, bid == 0);
-    }
-  }
-  auto group_offset = [&](int i) { return routed ? rt_off[i] : p.offsets[i]; };
   int g = bid / n_blocks;
   const int nb = bid - g * n_blocks;
   int mb = 0, me = p.M;
@@ -1031,8 +950,8 @@ __device__ __forceinline__ void skinny_gemm_body(const GemmArgs& p, int n_blocks
       const int gi = base + lane;
       int lo = 0, hi = 0;
       if (gi < G) {
-        lo = min(max(group_offset(gi), 0), p.M);
-        hi = min(max(group_offset(gi + 1), lo), p.M);
+        lo = min(max(p.offsets[gi], 0), p.M);
+        hi = min(max(p.offsets[gi + 1], lo), p.M);
       }
       const bool busy = hi > lo;
       const uint64_t mask = __ballot(busy);
@@ -1113,7 +1032,7 @@ __device__ __forceinline__ void skinny_gemm_body(const GemmArgs& p, int n_blocks
     for (int mt = 0; mt < MT; ++mt) {
       const int m = m0 + mt * 32 + r32;
       const int mm = m < me ? m : m0;
-      int row = GATHER ? (routed ? rt_tok[mm] : p.a_rows[mm]) : mm;
+      int row = GATHER ? p.a_rows[mm] : mm;
       row = (row >= 0 && row < row_limit) ? row : 0;
       toff[mt] = (uint32_t)(((int64_t)row * p.lda + 8 * h + k_beg) * 2);
     }
@@ -1412,7 +1331,7 @@ static int launch_skinny_gemm(const GemmArgs& a, hipStream_t st) {
     }
   }
   if constexpr (SWIGLU) {
-    // Fewer than two 32-column workgroups per CU (a one-token step: 8 groups x
+    // Fewer than two 32-column workgroups per CU (a call with 8 rows: 8 groups x
     // 44): a CU's fetch rate bounds each workgroup's weight stream, so the CUs
     // that hold two set the launch time. 16-column units halve the bytes per
     // workgroup and spread them over the CUs more evenly. Measured on MI355X:
@@ -1477,11 +1396,6 @@ template <bool SWIGLU, bool GATHER, bool TILED>
 static int run_gemm_t(const GemmArgs& a, hipStream_t st) {
   // groups of at most 64 rows (decode): weight streaming kernel
   const int rows = a.max_group_rows > 0 ? std::min(a.max_group_rows, a.M) : a.M;
-  // routing in the prologue exists only in the small-group SwiGLU kernel with gathered rows
-  DSK_REQUIRE(a.rt_parts == nullptr ||
-                  (SWIGLU && GATHER && rows <= kSkinnyMaxRows && a.offsets != nullptr &&
-                   a.rt_T >= 1 && a.rt_T <= kRouteInGemmTokens && a.M <= kRouteInGemmSlots),
-              DSK_ERR_INVALID_ARG, "grouped GEMM: routing in the prologue needs a small SwiGLU step");
   if (rows <= kSkinnyMaxRows) return launch_skinny<SWIGLU, GATHER, TILED>(a, rows, st);
   if (mid_gemm_takes(a, SWIGLU)) return run_mid_gemm(a, SWIGLU, st);
 #ifndef DSK_GEMM_WIDE

@@ -16,7 +16,10 @@
 // the lanes of a group are added by a fixed DPP tree, so results are the same
 // on every run.
 #include "dsk_internal.hpp"
+#include "gemm_common.hpp"
+#include "route_token.hpp"
 
+#include <algorithm>
 #include <climits>
 
 namespace dsk {
@@ -125,6 +128,142 @@ __global__ __launch_bounds__(64) void linear_rows_kernel(RowsArgs a) {
   }
 }
 
+// -------------------------------------------------- routing + gate/up -------
+// Routing and the first GEMM of a one-token MoE step in one launch: h[s] =
+// silu(Wg x) * (Wu x) for the token's K experts (slot s: ascending expert) and the
+// always-on groups (slot K + x). One wave per 8 gate rows and the matching 8 up rows of one
+// group (a 64 KB unit at H = 2048); 1408 units over 256 CUs leave 6 on the fullest against
+// 5.5 on average. A wave routes the token itself, in registers (route_token, on the gate's
+// partial planes; the picks' bit mask gives the slot's expert), so nothing runs between the
+// gate and this kernel, and the waves of the always-on groups, which need no routing,
+// stream meanwhile. Workgroup 0 stores the routing for the kernels after it.
+//
+// A lane holds one row and every eighth chunk, so each load instruction covers eight whole
+// lines and the weights pass the caches once. (With a line per lane and its 8 rows in 8
+// instructions, as linear_rows_kernel reads them, a CU holds more lines than its L1 and
+// fetches them again: 26 us, and 55 with loads that bypass the caches.) Against the MFMA
+// kernel of small groups with the routing in its prologue, which this replaces at one
+// token: 22.2 -> 18.8 us; the layer, with the next kernel's reads in the same order,
+// 36.6 -> 31.6 us.
+// Lane (r8, c8)'s first 16 bytes of row n0 + r8 (n0 a multiple of 8) of a [N, K] weight:
+// chunk c8 of the row's 8-element chunks.
+template <bool TILED>
+__device__ __forceinline__ const uint16_t* slab_lane(const uint16_t* w, int K, int n0, int r8,
+                                                     int c8) {
+  if constexpr (TILED)
+    return w + (int64_t)(n0 / 32) * (K / 16) * 512 + (n0 % 32 + r8) * 8 + (c8 >> 1) * 512 +
+           (c8 & 1) * 256;
+  else
+    return w + (int64_t)(n0 + r8) * K + c8 * 8;
+}
+
+// Sum over the 8 lanes that hold one row (lanes 8 apart), in a fixed order; all get it.
+__device__ __forceinline__ float chunk_lanes_sum(float v) {
+  v += __shfl_xor(v, 8, 64);
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+struct TokenGemm1Args {
+  const float* parts;  // [n_parts][E] partial gate sums
+  int n_parts;
+  int64_t part_stride;
+  const float* bias;
+  const uint16_t* x;   // [H]
+  const uint16_t* w1;  // [E + nsh, 2 I, H], row-major or tiled
+  uint16_t* h;         // [K + nsh, I]
+  int E, K, nsh, H, I;
+  int32_t* idx;
+  float* w;
+  int32_t* counts;
+  int32_t* offsets;
+  int32_t* token_map;
+  int32_t* slot_of;
+};
+
+template <bool TILED>
+__global__ __launch_bounds__(64) void token_gemm1_kernel(TokenGemm1Args a) {
+  constexpr int kBatch = 8;  // steps of 64 K elements in flight: 16 KB of weights
+  const int lane = threadIdx.x;
+  const int units = a.I / kRowsPerGroup;
+  const int slot = blockIdx.x / units, n0 = (blockIdx.x - slot * units) * kRowsPerGroup;
+  int g = a.E + slot - a.K;
+  if (slot < a.K) {  // uniform
+    int my_e;
+    float my_w;
+    // every 16-lane row of the wave routes the same token
+    route_token(a.parts, a.E, a.n_parts, a.part_stride, a.bias, 0, true, true, a.E, a.K, lane,
+                my_e, my_w);
+    uint64_t mask = 0;
+    for (int k = 0; k < a.K; ++k) mask |= 1ull << (__builtin_amdgcn_readlane(my_e, k) & 63);
+    uint64_t rest = mask;
+    for (int k = 0; k < slot; ++k) rest &= rest - 1;
+    g = __ffsll((unsigned long long)rest) - 1;
+    if (blockIdx.x == 0) {
+      if (lane < a.K) {
+        a.idx[lane] = my_e;
+        a.w[lane] = my_w;
+        a.slot_of[lane] = __popcll(mask & ((1ull << (my_e & 63)) - 1ull));
+      }
+      if (lane < a.E) {
+        a.offsets[lane] = __popcll(mask & ((1ull << lane) - 1ull));
+        a.counts[lane] = (int)((mask >> lane) & 1);
+      }
+      for (int i = lane; i <= a.nsh; i += 64) a.offsets[a.E + i] = a.K + i;
+      for (int i = lane; i < a.K + a.nsh; i += 64) a.token_map[i] = 0;
+    }
+  }
+  // lane = (row lane % 8, chunk lane / 8 of each step's 8): a load instruction covers eight
+  // whole 128-byte lines in either layout
+  const int r8 = lane & 7, c8 = lane >> 3;
+  const int steps = a.H / 64;
+  const uint16_t* base = a.w1 + (int64_t)g * 2 * a.I * a.H;
+  const uint16_t* gate = slab_lane<TILED>(base, a.H, n0, r8, c8);
+  const uint16_t* up = slab_lane<TILED>(base, a.H, a.I + n0, r8, c8);
+  const uint16_t* x = a.x + c8 * 8;
+  constexpr int kStep = TILED ? 2048 : 64;  // elements per 8 chunks
+  float ag = 0.f, au = 0.f;
+  for (int j0 = 0; j0 < steps; j0 += kBatch) {
+    u32x4_t wg[kBatch], wu[kBatch], xv[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int j = min(j0 + u, steps - 1);  // past the row: reload, unused
+      wg[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(gate + j * kStep));
+      wu[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(up + j * kStep));
+      xv[u] = *reinterpret_cast<const u32x4_t*>(x + j * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load of the batch before the first use
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (j0 + u < steps) {
+        ag = dot8(wg[u], xv[u], ag);
+        au = dot8(wu[u], xv[u], au);
+      }
+    }
+  }
+  ag = chunk_lanes_sum(ag);
+  au = chunk_lanes_sum(au);
+  if (c8 == 0) a.h[(int64_t)slot * a.I + n0 + r8] = f32_to_bf16(silu_f(ag) * au);
+}
+
+int launch_token_gemm1(const float* parts, int n_parts, int64_t part_stride, const float* bias,
+                       const uint16_t* x, const uint16_t* w1, bool tiled, uint16_t* h, int E,
+                       int K, int nsh, int H, int I, int32_t* idx, float* w, int32_t* counts,
+                       int32_t* offsets, int32_t* token_map, int32_t* slot_of, hipStream_t st) {
+  DSK_REQUIRE(n_parts >= 1 && n_parts <= kMaxGateParts && E >= 1 && E <= 64 && K >= 1 &&
+                  K <= std::min(E, 16) && nsh >= 0 && H % 64 == 0 && I % 32 == 0,
+              DSK_ERR_INVALID_ARG, "token_gemm1: sizes out of range");
+  const TokenGemm1Args a{parts, n_parts, part_stride, bias, x, w1, h, E, K, nsh, H, I,
+                         idx, w, counts, offsets, token_map, slot_of};
+  const dim3 grid((unsigned)((K + nsh) * (I / kRowsPerGroup)));
+  if (tiled)
+    hipLaunchKernelGGL(token_gemm1_kernel<true>, grid, dim3(64), 0, st, a);
+  else
+    hipLaunchKernelGGL(token_gemm1_kernel<false>, grid, dim3(64), 0, st, a);
+  return check_launch("token_gemm1_kernel");
+}
+
 // ------------------------------------------- down projection + combine ----
 // The MoE layer's second GEMM and its combine in one launch, for the smallest steps:
 //
@@ -138,14 +277,14 @@ __global__ __launch_bounds__(64) void linear_rows_kernel(RowsArgs a) {
 // (4.6 us) for 32 KB. Both are one launch if a workgroup has the same columns of every
 // busy group, and the even split of the columns also gives each CU the same bytes: a
 // workgroup owns 8 columns (one 128-byte line of each fragment half, as above), each of its
-// 8 waves takes every eighth busy group, all weight loads of a 1408-long row in flight at
-// once, and the rows of y meet in LDS. The layer at one token 39.0 -> 36.6 us, at two
-// tokens with 9 busy groups 49 -> 44 and with 13 58 -> 58. From three tokens up a wave's
-// bursts over several groups no longer fill the CU's queue (three tokens with 17 to 19 busy
-// groups 76 -> 79 us, four 82 -> 93), so larger steps keep the two launches.
+// 8 waves takes every eighth busy group, 11 KB of its rows in flight at once, and the rows
+// of y meet in LDS. The layer at one token 39.0 -> 36.6 us by this launch alone (with a line
+// per lane), at two tokens with 9 busy groups 49 -> 43 and with 13 58 -> 55. From three
+// tokens up a wave's bursts over several groups no longer fill the CU's queue (three tokens
+// 75 -> 77 us, four 80 -> 86), so larger steps keep the two launches.
 constexpr int kCombineWavesG2 = 8;
 constexpr int kCombineCols = 8;
-constexpr int kG2Batch = 3;    // 8-element K chunks per lane in flight (1408 = 2.75 x 512)
+constexpr int kG2Batch = 11;   // steps of 64 K elements in flight (1408 = 22 x 64)
 constexpr int kG2MaxSlots = 256;
 constexpr int kG2MaxK = 8;
 
@@ -165,7 +304,9 @@ __global__ __launch_bounds__(64 * kCombineWavesG2) void gemm2_combine_kernel(Gem
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * kCombineCols;
-  const int nch = a.I / 8;
+  const int r8 = lane & 7, c8 = lane >> 3;  // row and chunk of a lane, as above
+  const int steps = a.I / 64;
+  constexpr int kStep = TILED ? 2048 : 64;
 
   // busy groups, lane = group (G <= 128: two halves)
   int lo0 = 0, hi0 = 0, lo1 = 0, hi1 = 0;
@@ -202,51 +343,34 @@ __global__ __launch_bounds__(64 * kCombineWavesG2) void gemm2_combine_kernel(Gem
     const int g = src + (upper ? 64 : 0);
     const int lo = __builtin_amdgcn_readlane(upper ? lo1 : lo0, src);
     const int rows = min(__builtin_amdgcn_readlane(upper ? hi1 : hi0, src) - lo, MT);
-    const uint16_t* wb = a.w2 + (int64_t)g * a.H * a.I;
-    wb += TILED ? (int64_t)(n0 / 32) * (a.I / 16) * 512 + (n0 % 32 / kCombineCols) * 64
-                : (int64_t)n0 * a.I;
-    float acc[MT][kCombineCols];
+    const uint16_t* wb = slab_lane<TILED>(a.w2 + (int64_t)g * a.H * a.I, a.I, n0, r8, c8);
+    const uint16_t* hb = a.h + (int64_t)lo * a.I + c8 * 8;
+    float acc[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int i = 0; i < kCombineCols; ++i) acc[m][i] = 0.f;
-    for (int j0 = 0; j0 < nch; j0 += 64 * kG2Batch) {
-      u32x4_t wv[kG2Batch][kCombineCols], xv[kG2Batch][MT];
+    for (int m = 0; m < MT; ++m) acc[m] = 0.f;
+    for (int j0 = 0; j0 < steps; j0 += kG2Batch) {
+      u32x4_t wv[kG2Batch], xv[kG2Batch][MT];
 #pragma unroll
       for (int u = 0; u < kG2Batch; ++u) {
-        const int c = min(j0 + 64 * u + lane, nch - 1);  // past the row: reload, unused
-        const uint16_t* wp = TILED ? wb + (c >> 1) * 512 + (c & 1) * 256 : wb + c * 8;
-#pragma unroll
-        for (int i = 0; i < kCombineCols; ++i)
-          wv[u][i] = *reinterpret_cast<const u32x4_t*>(wp + (int64_t)i * (TILED ? 8 : a.I));
+        const int j = min(j0 + u, steps - 1);  // past the row: reload, unused
+        wv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wb + j * kStep));
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          xv[u][m] = *reinterpret_cast<const u32x4_t*>(a.h + (int64_t)(lo + min(m, rows - 1)) * a.I +
-                                                       c * 8);
+          xv[u][m] = *reinterpret_cast<const u32x4_t*>(hb + (int64_t)min(m, rows - 1) * a.I + j * 64);
       }
       __builtin_amdgcn_sched_barrier(0);  // every load of the batch before the first use
 #pragma unroll
       for (int u = 0; u < kG2Batch; ++u) {
-        if (j0 + 64 * u + lane < nch) {
+        if (j0 + u < steps) {
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int i = 0; i < kCombineCols; ++i)
-              acc[m][i] = dot8(wv[u][i], xv[u][m], acc[m][i]);
+          for (int m = 0; m < MT; ++m) acc[m] = dot8(wv[u], xv[u][m], acc[m]);
         }
       }
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      if (m < rows) {  // uniform
-        float v[kCombineCols];
-#pragma unroll
-        for (int i = 0; i < kCombineCols; ++i) v[i] = bf16_to_f32(f32_to_bf16(wave_sum(acc[m][i])));
-        if (lane == 0) {
-#pragma unroll
-          for (int i = 0; i < kCombineCols; ++i) s_y[lo + m][i] = v[i];
-        }
-      }
+      const float v = bf16_to_f32(f32_to_bf16(chunk_lanes_sum(acc[m])));
+      if (m < rows && c8 == 0) s_y[lo + m][r8] = v;
     }
   }
   // fixed sorting network on compile-time indices
@@ -272,7 +396,7 @@ __global__ __launch_bounds__(64 * kCombineWavesG2) void gemm2_combine_kernel(Gem
 
 bool gemm2_combine_takes(int T, int K, int G, int nsh, int H, int I) {
   return T >= 1 && T <= kGemm2CombineTokens && K <= kG2MaxK && G <= 128 &&
-         T * (K + nsh) <= kG2MaxSlots && H % 32 == 0 && I % 16 == 0;
+         T * (K + nsh) <= kG2MaxSlots && H % 32 == 0 && I % 64 == 0;
 }
 
 int launch_gemm2_combine(const uint16_t* h, const uint16_t* w2, bool tiled,

@@ -102,16 +102,9 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
     return DSK_OK;
   };
   int rc;
-  // Decode steps of at most kRouteInGemmTokens tokens: GEMM1's prologue does the
-  // routing (every workgroup for itself, workgroup 0 storing the results), so
-  // no route launch runs before it.
-#ifndef DSK_ROUTE_IN_GEMM
-#define DSK_ROUTE_IN_GEMM 1
-#endif
-  const bool route_in_gemm = DSK_ROUTE_IN_GEMM && nblk == 1 && T <= kRouteInGemmTokens &&
-                             Stot <= kRouteInGemmSlots &&
-                             n_parts >= 1 && n_parts <= kMaxGateParts;
-  if (route_in_gemm) {
+  // A one-token step is routed inside its first GEMM's launch.
+  const bool one_token = T == 1;
+  if (one_token) {
     // nothing to launch here
   } else if (nblk == 1) {
     rc = launch_route(logits, E, n_parts, part_stride, bias, T, E, K, idx, w, hist, rank,
@@ -128,35 +121,27 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
 
   if ((rc = mark(1))) return rc;
 
-  GemmArgs g1{};
-  g1.A = x; g1.lda = H;
-  g1.a_rows = token_map; g1.a_rows_limit = T;
-  g1.B = w1; g1.ldb = H; g1.b_group_stride = (int64_t)2 * I * H;
-  g1.C = h; g1.ldc = I;
-  g1.offsets = offsets; g1.G = G;
-  g1.M = Stot; g1.N = I; g1.K = H;
-  g1.offsets_sorted = 1;  // the route kernels' offsets never decrease
-  g1.up_row_offset = I;
-  g1.max_group_rows = T;  // a token routes to an expert at most once; shared groups hold T
-  g1.b_tiled = weight_layout == DSK_LAYOUT_TILED;
-  g1.chunk_m_tiles = group_chunk_m_tiles(T, E, K, nsh);
-  if (route_in_gemm) {
-    g1.rt_parts = logits;
-    g1.rt_n_parts = n_parts;
-    g1.rt_part_stride = part_stride;
-    g1.rt_bias = bias;
-    g1.rt_T = T;
-    g1.rt_E = E;
-    g1.rt_K = K;
-    g1.rt_nsh = nsh;
-    g1.rt_idx = idx;
-    g1.rt_w = w;
-    g1.rt_counts = counts;
-    g1.rt_offsets = offsets;
-    g1.rt_token_map = token_map;
-    g1.rt_slot_of = slot_of;
+  const int chunk_m_tiles = group_chunk_m_tiles(T, E, K, nsh);
+  if (one_token) {
+    rc = launch_token_gemm1(logits, n_parts, part_stride, bias, x, w1,
+                            weight_layout == DSK_LAYOUT_TILED, h, E, K, nsh, H, I, idx, w, counts,
+                            offsets, token_map, slot_of, st);
+    if (rc) return rc;
+  } else {
+    GemmArgs g1{};
+    g1.A = x; g1.lda = H;
+    g1.a_rows = token_map; g1.a_rows_limit = T;
+    g1.B = w1; g1.ldb = H; g1.b_group_stride = (int64_t)2 * I * H;
+    g1.C = h; g1.ldc = I;
+    g1.offsets = offsets; g1.G = G;
+    g1.M = Stot; g1.N = I; g1.K = H;
+    g1.offsets_sorted = 1;  // the route kernels' offsets never decrease
+    g1.up_row_offset = I;
+    g1.max_group_rows = T;  // a token routes to an expert at most once; shared groups hold T
+    g1.b_tiled = weight_layout == DSK_LAYOUT_TILED;
+    g1.chunk_m_tiles = chunk_m_tiles;
+    if ((rc = run_gemm(g1, true, st))) return rc;
   }
-  if ((rc = run_gemm(g1, true, st))) return rc;
   if ((rc = mark(2))) return rc;
 
   if (gemm2_combine_takes(T, K, G, nsh, H, I)) {
@@ -174,7 +159,7 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
     g2.offsets_sorted = 1;
     g2.max_group_rows = T;
     g2.b_tiled = weight_layout == DSK_LAYOUT_TILED;
-    g2.chunk_m_tiles = g1.chunk_m_tiles;
+    g2.chunk_m_tiles = chunk_m_tiles;
     if ((rc = run_gemm(g2, false, st))) return rc;
     if ((rc = mark(3))) return rc;
 
