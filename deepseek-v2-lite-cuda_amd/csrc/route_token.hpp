@@ -1,6 +1,6 @@
 // Softmax and top-K selection of one token on a 16-lane row, shared by the
-// route kernel (moe_route.hip) and the small-group GEMM that routes a decode
-// step in its prologue (gemm.hip), so both pick the same experts with the same
+// route kernel (moe_route.hip) and the first GEMM of a one-token step, which
+// routes for itself (gemv.hip), so both pick the same experts with the same
 // weights, bit for bit.
 #pragma once
 
