@@ -234,8 +234,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
     const int nblk = (gme - mb + 31) / 32;
     int nt, mi;
     sched_group_tile(local, mt, NT, &nt, &mi);
-    const int m0 = mb + 32 * (mi * nblk / mt);
-    const int me = min(mb + 32 * ((mi + 1) * nblk / mt), gme);
+    const int m0 = mb + 32 * sched_tile_block(mi, mt, nblk, BM / 32);
+    const int me = min(mb + 32 * sched_tile_block(mi + 1, mt, nblk, BM / 32), gme);
     return Tile{lo, m0, me, nt * OUT_N};
   };
 
@@ -627,8 +627,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
     const int nblk = (gme - mb + 31) / 32;
     int nt, mi;
     sched_group_tile(local, mt, NT, &nt, &mi);
-    const int m0 = mb + 32 * (mi * nblk / mt);
-    const int me = min(mb + 32 * ((mi + 1) * nblk / mt), gme);
+    const int m0 = mb + 32 * sched_tile_block(mi, mt, nblk, TM);
+    const int me = min(mb + 32 * sched_tile_block(mi + 1, mt, nblk, TM), gme);
     return Tile{lo, m0, me, nt * OUT_N};
   };
 

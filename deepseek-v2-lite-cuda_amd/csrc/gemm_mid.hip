@@ -75,8 +75,8 @@ __device__ __forceinline__ void mid_tile(const GemmArgs& p, int W, int NT, char*
   int nt, mi;
   sched_group_tile(local, mt, NT, &nt, &mi);
   nt = __builtin_amdgcn_readfirstlane(nt);
-  const int m0 = __builtin_amdgcn_readfirstlane(mb + 32 * (mi * nblk / mt));
-  const int me = __builtin_amdgcn_readfirstlane(min(mb + 32 * ((mi + 1) * nblk / mt), gme));
+  const int m0 = __builtin_amdgcn_readfirstlane(mb + 32 * sched_tile_block(mi, mt, nblk, TM));
+  const int me = __builtin_amdgcn_readfirstlane(min(mb + 32 * sched_tile_block(mi + 1, mt, nblk, TM), gme));
   const int n0 = nt * OUT_N;
   const int tma = (me - m0 + 31) / 32;  // token blocks with rows
   const int nk = p.K / kMidBK;

@@ -93,6 +93,15 @@ DSK_HD void sched_group_tile(int local, int mt, int nt_count, int* nt, int* mi) 
   *mi = p * kPanelM + (r - *nt * ps);
 }
 
+// First 32-row block of M tile mi when a group's nblk blocks are split evenly over its
+// mt = ceil(nblk / tm) tiles of at most tm blocks: floor(mi * nblk / mt). That product
+// passes 2^31 from 2.1 million rows in tiles of two blocks, so it is taken apart:
+// nblk = mt * tm - spare with spare < tm.
+DSK_HD int sched_tile_block(int mi, int mt, int nblk, int tm) {
+  const int spare = mt * tm - nblk;
+  return mi * tm - (mi * spare + mt - 1) / mt;
+}
+
 // The largest number of tiles any workgroup runs (nwg a multiple of 8).
 DSK_HD int sched_max_tiles(int total, int nwg, int chunk) {
   int m = 0;

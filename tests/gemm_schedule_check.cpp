@@ -8,6 +8,8 @@
 //      real tile count (which the launcher bounds from above).
 //   3. A group's tile order (panels of M tiles) maps its local tile indices
 //      onto its (N tile, M tile) pairs one to one.
+//   4. The even split of a group's 32-row blocks over its M tiles covers the blocks in
+//      order, at most a tile's worth each, up to the most rows an operand of 4 GiB has.
 #include <cstdio>
 #include <cstdlib>
 #include <algorithm>
@@ -89,6 +91,22 @@ int main() {
         if (nt < 0 || nt >= nc || mi < 0 || mi >= mt) return fail("group tile out of range", mt, nc, l);
         if (seen[mi * nc + nt]++) return fail("group tile run twice", mt, nc, l);
       }
+    }
+  }
+  // 4. the row split, against the same in 64 bits
+  for (int tm : {2, 4, 8}) {
+    for (long long rows = 1; rows <= 33554432; rows += rows < 5000 ? 1 : rows / 3 + 17) {
+      const int nblk = (int)((rows + 31) / 32), mt = (int)((rows + 32 * tm - 1) / (32 * tm));
+      const int step = mt > 20000 ? 61 : 1;
+      for (int mi = 0; mi <= mt; mi += mi + step <= mt || mi == mt ? step : mt - mi) {
+        const int b = sched_tile_block(mi, mt, nblk, tm);
+        if (b != (long long)mi * nblk / mt) return fail("row split", rows, tm, mi);
+        if (mi < mt) {
+          const int n = sched_tile_block(mi + 1, mt, nblk, tm) - b;
+          if (n < 1 || n > tm) return fail("blocks of a tile", rows, tm, mi);
+        }
+      }
+      if (sched_tile_block(mt, mt, nblk, tm) != nblk) return fail("row split end", rows, tm, mt);
     }
   }
   std::printf("OK\n");

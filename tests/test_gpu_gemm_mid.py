@@ -45,6 +45,18 @@ def test_dense(dsk, M, N, K):
     assert bool((guard[0] == 7).all() and (guard[M + 1] == 7).all() and (guard[:, N:] == 7).all())
 
 
+# rows times blocks past 2^31: 64-row tiles from 2.1 million rows, 128-row ones from 3.0
+@pytest.mark.parametrize("M,N", [(2200003, 128), (3100003, 256)])
+def test_dense_millions_of_rows(dsk, M, N):
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(M, 64, generator=g, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(N, 64, generator=g, device=DEV).mul_(0.05).to(torch.bfloat16)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    dsk.linear(x, dsk.tile_weights(w[None])[0], out=out)
+    for r in range(0, M, 400000):
+        _check(out[r:r + 400000], x[r:r + 400000], w)
+
+
 @pytest.mark.parametrize("M", [1, 33, 64, 200, 777, 1111, 4100])
 def test_row_statistics(dsk, M):
     """linear_rowsq / linear_rowscale on 64- and 128-row tiles."""
