@@ -519,14 +519,39 @@ __global__ __launch_bounds__(256) void combine_lists_kernel(
 // The generic combine in one launch, while reading the token map in every workgroup is
 // cheap: a workgroup owns two tokens, collects their slots from the whole map, puts each
 // list in ascending order by counting and sums the rows, two waves per token, in the order
-// and arithmetic of combine_lists_kernel. A token with more slots than a list holds walks
-// the map instead. Replaces five launches (T = 600, S = 3600: 25.8 -> 7.6 us).
+// and arithmetic of combine_lists_kernel. Replaces five launches: top-6 maps through the
+// op, T = 600 27.0 -> 12.9 us, 2000 26.5 -> 14.0, 3344 31.5 -> 23.0.
+//
+// A token with more slots than a list holds walks the map again, 1024 slots at a time in
+// ascending order, and adds the rows as a ballot finds them (one of 512 tokens with 1500 of
+// 3072 slots: 461 us, the five launches 1077; with a dependent load per slot it took 1123).
 constexpr int kCombineTokens = 2;
 constexpr int kCombineWaves = 2;   // per token
-constexpr int kCombineList = 64;
-// bytes of the map read by all workgroups up to which this is the faster one (48 MB: 14 us
-// through the op, the five launches 27)
+constexpr int kCombineList = 128;
+// Where the map is read this way: bytes of it read by all workgroups (at the line, T = 3344,
+// 23.0 against 31.5 us. Past it this kernel is still ahead at 192 MB, T = 4096, 26.3 against
+// 34.8, and nothing further was measured)...
 constexpr int64_t kCombineScanBytes = (int64_t)128 << 20;
+// ...and slots per token on average: up to half a list, so that uneven maps overflow few
+// lists. Random maps of 512 tokens through the op, us, this kernel / five launches: 6 slots
+// each 13 / 24, 16 15 / 28, 32 26 / 49, 48 36 / 66, 64 43 / 81; 88, past the line, 63 / 107,
+// and 128, where half the tokens walk, 274 / 154.
+constexpr int kCombineScanMean = 64;
+
+// acc[0..8) += wt * the 8 bf16 of v, and the 8 sums rounded to bf16
+__device__ __forceinline__ void add_row(float wt, const u32x4_t& v, float (&acc)[8]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    acc[2 * j] = fmaf(wt, bf16lo(v[j]), acc[2 * j]);
+    acc[2 * j + 1] = fmaf(wt, bf16hi(v[j]), acc[2 * j + 1]);
+  }
+}
+__device__ __forceinline__ u32x4_t pack_row(const float (&acc)[8]) {
+  u32x4_t o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
+  return o;
+}
 
 __global__ __launch_bounds__(64 * kCombineTokens * kCombineWaves) void combine_scan_kernel(
     const uint16_t* __restrict__ y, const int32_t* __restrict__ token_map,
@@ -559,48 +584,78 @@ __global__ __launch_bounds__(64 * kCombineTokens * kCombineWaves) void combine_s
   }
   __syncthreads();
   const int n = s_n[r];
-  if (part == 0 && n <= kCombineList && lane < n) {
-    const int v = s_list[r][lane];
-    const float wt = dw[v];
-    int at = 0;
-    for (int j = 0; j < n; ++j) at += s_list[r][j] < v;
-    s_sorted[r][at] = v;
-    s_w[r][at] = wt;
+  if (part == 0 && n <= kCombineList) {
+    for (int i = lane; i < n; i += 64) {
+      const int v = s_list[r][i];
+      const float wt = dw[v];
+      int at = 0;
+      for (int j = 0; j < n; ++j) at += s_list[r][j] < v;
+      s_sorted[r][at] = v;
+      s_w[r][at] = wt;
+    }
   }
   __syncthreads();
   const int tok = t0 + r;
   if (tok >= T) return;
+  constexpr int R = 6;  // rows in flight
+  if (n > kCombineList) {  // uniform over the wave, whose lanes all take part in the walk
+    for (int c0 = 64 * part; c0 < H / 8; c0 += 64 * kCombineWaves) {
+      const int c = min(c0 + lane, H / 8 - 1);
+      float acc[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+      for (int s0 = 0; s0 < S; s0 += 64 * U) {
+        int t[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int s = s0 + 64 * u + lane;
+          t[u] = s < S ? token_map[s] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          uint64_t m = __ballot(t[u] == tok);
+          while (m != 0) {
+            int slot[R];
+            bool on[R];
+            u32x4_t v[R];
+            float wt[R];
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+              on[q] = m != 0;
+              slot[q] = on[q] ? s0 + 64 * u + __ffsll((unsigned long long)m) - 1 : slot[0];
+              m &= m - 1;
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+              wt[q] = dw[slot[q]];
+              v[q] = reinterpret_cast<const u32x4_t*>(y + (int64_t)slot[q] * H)[c];
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+              if (on[q]) add_row(wt[q], v[q], acc);
+          }
+        }
+      }
+      if (c0 + lane < H / 8) reinterpret_cast<u32x4_t*>(out + (int64_t)tok * H)[c] = pack_row(acc);
+    }
+    return;
+  }
 #pragma unroll 2
   for (int c = 64 * part + lane; c < H / 8; c += 64 * kCombineWaves) {
     float acc[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.f;
-    auto add = [&](float wt, const u32x4_t& v) {
+    for (int i = 0; i < n; i += R) {
+      u32x4_t v[R];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[2 * j] = fmaf(wt, bf16lo(v[j]), acc[2 * j]);
-        acc[2 * j + 1] = fmaf(wt, bf16hi(v[j]), acc[2 * j + 1]);
-      }
-    };
-    auto row = [&](int s) { return reinterpret_cast<const u32x4_t*>(y + (int64_t)s * H)[c]; };
-    if (n <= kCombineList) {
-      constexpr int R = 6;  // rows in flight
-      for (int i = 0; i < n; i += R) {
-        u32x4_t v[R];
+      for (int u = 0; u < R; ++u)
+        v[u] = reinterpret_cast<const u32x4_t*>(
+            y + (int64_t)s_sorted[r][min(i + u, n - 1)] * H)[c];
 #pragma unroll
-        for (int u = 0; u < R; ++u) v[u] = row(s_sorted[r][min(i + u, n - 1)]);
-#pragma unroll
-        for (int u = 0; u < R; ++u)
-          if (i + u < n) add(s_w[r][i + u], v[u]);
-      }
-    } else {
-      for (int s = 0; s < S; ++s)
-        if (token_map[s] == tok) add(dw[s], row(s));
+      for (int u = 0; u < R; ++u)
+        if (i + u < n) add_row(s_w[r][i + u], v[u], acc);
     }
-    u32x4_t o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
-    reinterpret_cast<u32x4_t*>(out + (int64_t)tok * H)[c] = o;
+    reinterpret_cast<u32x4_t*>(out + (int64_t)tok * H)[c] = pack_row(acc);
   }
 }
 
@@ -853,7 +908,8 @@ extern "C" int dsk_moe_combine(const dsk_bf16* expert_out, const int32_t* token_
               DSK_ERR_WORKSPACE, "moe_combine: workspace too small");
   hipStream_t st = as_stream(stream);
   const int64_t groups = ((int64_t)num_tokens + kCombineTokens - 1) / kCombineTokens;
-  if (groups * total_slots * (int64_t)sizeof(int32_t) <= kCombineScanBytes) {
+  if (groups * total_slots * (int64_t)sizeof(int32_t) <= kCombineScanBytes &&
+      total_slots <= (int64_t)kCombineScanMean * num_tokens) {
     hipLaunchKernelGGL(combine_scan_kernel, dim3((unsigned)groups),
                        dim3(64 * kCombineTokens * kCombineWaves), 0, st, expert_out, token_map,
                        dispatched_weights, total_slots, num_tokens, hidden, out);
