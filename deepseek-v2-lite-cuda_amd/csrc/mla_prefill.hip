@@ -142,18 +142,21 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillArgs a)
   const uint32_t c_v = (uint32_t)((lane & 15) ^ (row4 << 2)) * 16 + kPfNope * 2;
   const uint32_t c_r = (uint32_t)((lane & 7) ^ row8 ^ (wave & 1)) * 16;
   auto dma_tile = [&](int t, uint32_t buf) __attribute__((always_inline)) {
-    const int k0 = t * kPfTile;
+    // 64-bit base of the tile, 32-bit offsets inside it: a sequence may span any size
+    const int k0 = t * kPfTile, last = a.L - 1 - k0;
+    const char* kv_t = kv_b + (int64_t)k0 * ldkv2;
+    const char* kr_t = kr_b + (int64_t)k0 * ldkr2;
 #pragma unroll
     for (int j = 0; j < 16 / NW; ++j) {
       const int i = wave + NW * j;
-      const uint32_t row = (uint32_t)min(k0 + 4 * i + row4, a.L - 1) * ldkv2;
-      dma_1kb(kv_b, row + c_k, buf + i * 1024);
-      dma_1kb(kv_b, row + c_v, buf + kPfVOff + i * 1024);
+      const uint32_t row = (uint32_t)min(4 * i + row4, last) * ldkv2;
+      dma_1kb(kv_t, row + c_k, buf + i * 1024);
+      dma_1kb(kv_t, row + c_v, buf + kPfVOff + i * 1024);
     }
 #pragma unroll
     for (int j = 0; j < 8 / NW; ++j) {
       const int i = wave + NW * j;
-      dma_1kb(kr_b, (uint32_t)min(k0 + 8 * i + row8, a.L - 1) * ldkr2 + c_r,
+      dma_1kb(kr_t, (uint32_t)min(8 * i + row8, last) * ldkr2 + c_r,
               buf + kPfRopeOff + i * 1024);
     }
   };
@@ -371,10 +374,10 @@ extern "C" int dsk_mla_prefill_attention(
                   ld_kr >= kPfRope && ld_cs >= kPfRope && ld_out >= (int64_t)heads * kPfV &&
                   kr_batch_stride >= 0 && cs_batch_stride >= 0,
               DSK_ERR_INVALID_ARG, "mla_prefill_attention: row stride smaller than the row");
-  // one sequence's keys are addressed by 32-bit byte offsets
-  DSK_REQUIRE((int64_t)kv_len * ld_kv * 2 < ((int64_t)1 << 32) &&
-                  (int64_t)kv_len * ld_kr * 2 < ((int64_t)1 << 32),
-              DSK_ERR_INVALID_ARG, "mla_prefill_attention: one sequence must span less than 4 GiB");
+  // the rows of one tile are addressed by 32-bit byte offsets
+  const int64_t tile_rows = std::min(kv_len, kPfTile);
+  DSK_REQUIRE(tile_rows * ld_kv * 2 < ((int64_t)1 << 32) && tile_rows * ld_kr * 2 < ((int64_t)1 << 32),
+              DSK_ERR_INVALID_ARG, "mla_prefill_attention: 64 key rows must span less than 4 GiB");
   DSK_REQUIRE((int64_t)batch * heads <= INT32_MAX && q_len <= 65535 * 128, DSK_ERR_INVALID_ARG,
               "mla_prefill_attention: too many query blocks");
   PrefillArgs a;

@@ -442,3 +442,4 @@ def test_prefill_attention_validation(dsk):
     assert call(q=None) == 2
     assert call(q=8) == 3 and call(ld_q=3076) == 3 and call(ld_out=2052) == 3
     assert call(ld_q=3064) == 1 and call(ld_kv=4088) == 1 and call(ld_kr=56) == 1
+    assert call(L=64, ld_kv=1 << 25) == 1 and call(L=64, ld_kr=1 << 25) == 1 and "4 GiB" in _err(dsk)

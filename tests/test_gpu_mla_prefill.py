@@ -72,6 +72,16 @@ def test_causal(dsk, b, n, L, heads):
     assert torch.equal(out, dsk.mla_prefill_attention(*ops_in, SCALE, heads=heads))
 
 
+def test_sequence_of_more_than_4_gib(dsk):
+    """Key rows 16 KB apart: 270000 of them span 4.4 GB."""
+    n, L, heads = 40, 270000, 2
+    q, _, kr, cos, sin = _operands(1, n, L, heads, 11)
+    kv = torch.empty(1, L, 8192, dtype=torch.bfloat16, device=DEV)[..., :heads * 256]
+    kv.copy_(torch.randn(1, L, heads * 256, device=DEV))
+    out = dsk.mla_prefill_attention(q, kv, kr, cos, sin, SCALE, heads=heads)
+    _check(out, *_reference(q, kv, kr, cos, sin, heads, True, None))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", ["b1qk", "bhqk", "11qk", "k", "bhqk_strided"])
 @pytest.mark.parametrize("b,n,L", [(2, 70, 77), (16, 130, 131)])
