@@ -209,6 +209,11 @@ UP_PROJECTED_MIN_TOKENS = 128
 # Largest decode step (new tokens of all sequences) that runs as one C call.
 NATIVE_MAX_TOKENS = 64
 
+# Steps that do not (other head dims, weights that are only partly tiled) run their
+# projections on the vector-ALU row kernel (dsk_linear_rows) up to this many tokens, as
+# the C call does, and longer ones on the small-group MFMA kernel.
+ROWS_MAX_TOKENS = 4
+
 
 def _attend_up_projected(q: torch.Tensor, cache: LatentKVCache, W: MLAWeights, cos: torch.Tensor,
                          sin: torch.Tensor, eps: float) -> torch.Tensor:
@@ -309,18 +314,34 @@ def _decode_step(x: torch.Tensor, W: MLAWeights, cache: LatentKVCache, rows: tor
         return _decode_step_native(x.contiguous(), W, cache, cos.contiguous(), sin.contiguous(),
                                    A, eps)
     x2 = x.reshape(T, H)
-    q = ops.linear(x, W.q).view(T, h, nope + r)
-    if b == 1 or n == 1:                               # one row stride: project in place
-        ops.linear(x2, W.kva, out=rows[0] if b == 1 else rows[:, 0])
+    nq = h * (nope + r)
+    one_q_kva = W.q_kva is not None and W.q_kva.dim() == 4
+    few = (T <= ROWS_MAX_TOKENS and one_q_kva and W.o.dim() == 4 and A.uk_tiled is not None
+           and H % 128 == 0 and nope % 128 == 0)      # the row kernel's inner sizes
+    if (b == 1 or n == 1) and one_q_kva and T <= 64:
+        # q_proj and kv_a_proj in one launch, kv_a's rows straight into the slots
+        q = torch.empty((T, nq), dtype=torch.bfloat16, device=x.device)
+        dst = rows[0] if b == 1 else rows[:, 0]
+        if few:
+            ops.linear_rows(x2, W.q_kva, out=q, out1=dst, n_split=nq)
+        else:
+            ops.linear_split(x2, W.q_kva, q, dst)
+        q = q.view(T, h, nope + r)                         # [T, h, 192]
     else:
-        rows.copy_(ops.linear(x2, W.kva).view(b, n, lora + r))
+        q = ops.linear(x, W.q).view(T, h, nope + r)
+        if b == 1 or n == 1:                               # one row stride: project in place
+            ops.linear(x2, W.kva, out=rows[0] if b == 1 else rows[:, 0])
+        else:
+            rows.copy_(ops.linear(x2, W.kva).view(b, n, lora + r))
     L = cache.current_len
     if n >= UP_PROJECTED_MIN_TOKENS:
         o = _attend_up_projected(q.view(b, n, h, nope + r), cache, W, cos, sin, eps)
         return ops.linear(o, W.o)
     latent, k_pe = cache.get(L)
     small = T <= 64 and A.uk_tiled is not None
-    if small:   # per-head products on strided views, one launch each
+    if few:
+        q_abs = ops.linear_rows(q[..., :nope].transpose(0, 1), A.uk_tiled)     # [h, T, lora]
+    elif small:   # per-head products on strided views, one launch each
         q_abs = ops.linear_batched(q[..., :nope].transpose(0, 1), A.uk_tiled)  # [h, T, lora]
     else:
         q_abs = torch.bmm(q[..., :nope].transpose(0, 1).contiguous(), A.w_uk)
@@ -331,9 +352,12 @@ def _decode_step(x: torch.Tensor, W: MLAWeights, cache: LatentKVCache, rows: tor
     cache._rope_len = L          # the kernel rotated and stored the new keys
     if small:   # o[t, h*v:(h+1)*v] = o_lat[h, t] @ (W_UV[h] * w)^T, written token-major
         o = torch.empty((T, h * vd), dtype=torch.bfloat16, device=x.device)
-        ops.linear_batched(o_lat, A.uv_tiled, out=o.view(T, h, vd).transpose(0, 1))
+        (ops.linear_rows if few else ops.linear_batched)(o_lat, A.uv_tiled,
+                                                         out=o.view(T, h, vd).transpose(0, 1))
     else:
         o = torch.bmm(o_lat, A.w_uv_t).transpose(0, 1).reshape(T, h * vd)
+    if few:
+        return ops.linear_rows(o, W.o).view(b, n, -1)
     return ops.linear(o, W.o).view(b, n, -1)
 
 

@@ -89,3 +89,39 @@ def test_decode_step(setup, b, n):
         assert torch.equal(out, ref)
         assert torch.equal(caches[0].rows, caches[1].rows)
         assert caches[0].rope_len == caches[1].rope_len == L
+
+
+@pytest.mark.parametrize("dims", [(128, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("b,n,launches", [(1, 1, 4), (3, 1, 4), (1, 7, 1), (33, 1, 1)])
+def test_decode_step_op_by_op(monkeypatch, dims, b, n, launches):
+    """Steps that the C call does not take (other head dims; an o_proj that is not tiled) keep
+    the decode kernels: all projections on the row kernel up to 4 tokens where the weights are
+    tiled, q and kv_a in one launch up to 64. Against mla_forward on the whole sequence: bf16
+    roundings of the latent, of the absorbed weights and of four intermediates, 2e-2 as for
+    the other decode steps."""
+    import ds_kernels as dsk
+    from ds_kernels import mla as dm
+    from ds_kernels import ops
+    from ds_kernels import synthetic as syn
+    nope, vd = dims
+    w = syn.mla_weights(H=512, nope=nope, v_dim=vd)
+    W = dataclasses.replace(dm.MLAWeights.from_tensors(w, torch.device(DEV, 0)), nope=nope, v_dim=vd)
+    A = dsk.AbsorbedMLAWeights.from_mla(W)
+    if dims == (128, 128):
+        W = dataclasses.replace(W, o=dsk.untile_weights(W.o[None])[0])
+    if dims != (128, 64):     # the row kernel takes tiled weights with inner sizes of 128
+        launches = 1
+    cos, sin = (t.to(torch.bfloat16).to(DEV) for t in dm.yarn_cos_sin(64))
+    calls = []
+    for name in ("linear_rows", "linear_split"):
+        real = getattr(ops, name)
+        monkeypatch.setattr(ops, name,
+                            lambda *a, _f=real, _n=name, **k: (calls.append(_n), _f(*a, **k))[1])
+    x = _x(b, 20 + n, 512, seed=b + n)
+    cache = dsk.LatentKVCache.for_inference(b, max_seq=20 + n)
+    dsk.mla_decode_forward(x[:, :20], W, cache, cos, sin, A)
+    calls.clear()
+    out = dsk.mla_decode_forward(x[:, 20:].contiguous(), W, cache, cos, sin, A)
+    assert calls == (["linear_rows"] * 4 if launches == 4 else ["linear_split"])
+    ref = dm.mla_forward(x, W, cos, sin)[:, 20:].double()
+    assert float((out.double() - ref).abs().max() / ref.abs().max()) <= 2e-2
