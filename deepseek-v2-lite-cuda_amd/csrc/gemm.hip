@@ -1260,16 +1260,12 @@ static void allow_lds(std::once_flag (&once)[kMaxDevices], const void* kern, int
 }
 
 // Chunk and workgroups of a persistent launch of at most `upper` tiles of nt N tiles
-// each. Every XCD gets a workgroup per tile it holds, up to its CUs (fewer, and 15
-// tiles in one chunk of 16 would share two workgroups of one XCD).
+// each.
 static int64_t persistent_grid(GemmArgs& a, int64_t upper, int64_t nt, int row_tiles) {
   const int64_t cus = num_cus();
-  const int bound = (int)std::min<int64_t>(upper, INT32_MAX);
-  a.chunk = a.chunk_m_tiles > 0 ? sched_chunk(a.chunk_m_tiles, (int)nt)
-                                : sched_balanced_chunk(bound, (int)cus);
-  const int64_t xcd_tiles = sched_xcd_tiles(bound, 0, a.chunk);
-  return std::max(sched_workgroups(upper, cus, row_tiles, a.chunk),
-                  std::min(kXcds * xcd_tiles, cus / kXcds * kXcds));
+  a.chunk = sched_chunk(a.chunk_m_tiles, (int)nt, (int)std::min<int64_t>(upper, INT32_MAX),
+                        (int)cus);
+  return sched_persistent_workgroups(upper, cus, row_tiles, a.chunk);
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool SWIGLU,

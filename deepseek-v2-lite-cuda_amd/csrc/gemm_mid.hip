@@ -389,7 +389,7 @@ static int launch_mid(const GemmArgs& a, hipStream_t st) {
   if (tiles > INT32_MAX / 2)
     return fail(DSK_ERR_INVALID_ARG, "mid_gemm: too many tiles");
   const int chunk = sched_balanced_chunk((int)tiles, num_cus());
-  const int64_t grid = (tiles + kXcds * chunk - 1) / (kXcds * chunk) * (kXcds * chunk);
+  const int64_t grid = sched_single_workgroups(tiles, chunk);
   hipLaunchKernelGGL((mid_gemm_kernel<TM, TN, SWIGLU, GATHER, TILED>), dim3((unsigned)grid),
                      dim3(kMidThreads), 0, st, a, chunk);
   return check_launch("mid_gemm_kernel");

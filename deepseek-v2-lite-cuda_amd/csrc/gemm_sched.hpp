@@ -4,8 +4,8 @@
 // alone for the CPU check of the schedule (tests/gemm_schedule_check.cpp).
 //
 // A launch enumerates T output tiles (group-major, then N tile, then M tile)
-// and deals them to the 8 XCDs in chunks of `chunk` consecutive tiles (see
-// sched_chunk): chunk c goes to XCD c % 8, so every XCD gets the same mix of
+// and deals them to the 8 XCDs in chunks of `chunk` consecutive tiles (sched_chunk;
+// sched_balanced_chunk for the medium-problem kernel): chunk c goes to XCD c % 8, so every XCD gets the same mix of
 // tile sizes and the M tiles that share a weight tile stay on one XCD (one L2). Workgroup i
 // runs on XCD i % 8 in slot i / 8; inside an XCD, the XCD's q-th tile goes to
 // slot q % per_xcd in round q / per_xcd, so consecutive tiles run at the same
@@ -22,24 +22,21 @@
 
 namespace dsk {
 
-constexpr int kTileChunk = 16;  // tiles dealt to one XCD at a time, by default
+constexpr int kTileChunk = 16;  // most tiles dealt to one XCD at a time by the balanced deal
 constexpr int kXcds = 8;
 
-// Tiles per chunk: kTileChunk, or, when the caller knows the M tiles of a
-// typical group (chunk_m_tiles > 0), that many M tiles times the launch's nt N
-// tiles, so that one typical group's tiles go to one XCD and its token rows
-// are read into one L2. Measured on MI355X in the MoE layer at T = 4096
-// (routed groups of two M tiles): GEMM1 (11 N tiles) with chunks of 22 against
-// 16 ran 364.6 against 372.9 us and read 1.094 against 1.167 GB past the L2;
-// GEMM2 (8 N tiles) with chunks of 22 ran 246.4 against 210.7 us.
-DSK_HD int sched_chunk(int chunk_m_tiles, int nt) {
-  return chunk_m_tiles > 0 ? chunk_m_tiles * nt : kTileChunk;
+// Tiles held by XCD `xcd` out of `total`.
+DSK_HD int sched_xcd_tiles(int total, int xcd, int chunk) {
+  const int n_chunks = (total + chunk - 1) / chunk;
+  if (xcd >= n_chunks) return 0;
+  int t = ((n_chunks - xcd + kXcds - 1) / kXcds) * chunk;
+  if ((n_chunks - 1) % kXcds == xcd) t -= n_chunks * chunk - total;  // partial last chunk
+  return t;
 }
 
 // Chunk for a launch of `total` tiles on `cus` compute units: the largest of 16, 8, 4,
 // 2, 1 that leaves no XCD with more tiles per CU than an even deal would (a chunk of
 // 16 on 15 tiles would run all of them on one XCD).
-DSK_HD int sched_xcd_tiles(int total, int xcd, int chunk);
 DSK_HD int sched_balanced_chunk(int total, int cus) {
   const int per_xcd = cus / kXcds > 0 ? cus / kXcds : 1;
   const int even = (total + kXcds - 1) / kXcds;  // tiles of the fullest XCD at chunk 1
@@ -49,13 +46,14 @@ DSK_HD int sched_balanced_chunk(int total, int cus) {
   return 1;
 }
 
-// Tiles held by XCD `xcd` out of `total`.
-DSK_HD int sched_xcd_tiles(int total, int xcd, int chunk) {
-  const int n_chunks = (total + chunk - 1) / chunk;
-  if (xcd >= n_chunks) return 0;
-  int t = ((n_chunks - xcd + kXcds - 1) / kXcds) * chunk;
-  if ((n_chunks - 1) % kXcds == xcd) t -= n_chunks * chunk - total;  // partial last chunk
-  return t;
+// Tiles per chunk. When the caller knows the M tiles of a typical group (chunk_m_tiles > 0):
+// that many M tiles times the launch's nt N tiles, so that one typical group's tiles go to
+// one XCD and its token rows are read into one L2. Measured on MI355X in the MoE layer at
+// T = 4096 (routed groups of two M tiles): GEMM1 (11 N tiles) with chunks of 22 against
+// 16 ran 364.6 against 372.9 us and read 1.094 against 1.167 GB past the L2;
+// GEMM2 (8 N tiles) with chunks of 22 ran 246.4 against 210.7 us. Otherwise balanced.
+DSK_HD int sched_chunk(int chunk_m_tiles, int nt, int total, int cus) {
+  return chunk_m_tiles > 0 ? chunk_m_tiles * nt : sched_balanced_chunk(total, cus);
 }
 
 // Tiles run by workgroup slot `slot` of an XCD that holds xcd_tiles tiles over
@@ -127,6 +125,24 @@ inline int64_t sched_workgroups(int64_t upper, int64_t cus, int row_tiles, int c
     if (nwg < kXcds * per_xcd_min) nwg = kXcds * per_xcd_min;
   }
   return nwg;
+}
+
+// Workgroups of a persistent launch of at most `upper` tiles: sched_workgroups, and in every
+// XCD a workgroup per tile it holds, up to its CUs (fewer, and 15 tiles in one chunk of 16
+// would share two workgroups of one XCD).
+inline int64_t sched_persistent_workgroups(int64_t upper, int64_t cus, int row_tiles, int chunk) {
+  const int64_t bound = upper < INT32_MAX ? upper : INT32_MAX;
+  const int64_t by_tiles = (int64_t)kXcds * sched_xcd_tiles((int)bound, 0, chunk);
+  const int64_t by_cus = cus / kXcds * kXcds;
+  const int64_t a = sched_workgroups(upper, cus, row_tiles, chunk);
+  const int64_t b = by_tiles < by_cus ? by_tiles : by_cus;
+  return a > b ? a : b;
+}
+
+// Workgroups of a launch with one tile each: workgroup i runs tile
+// sched_tile_index(i & 7, i >> 3, 0, 1, chunk), whole chunks for every XCD.
+inline int64_t sched_single_workgroups(int64_t tiles, int chunk) {
+  return (tiles + kXcds * chunk - 1) / (kXcds * chunk) * (kXcds * chunk);
 }
 
 }  // namespace dsk

@@ -3,6 +3,8 @@
 // first failing case and exits non-zero.
 //   1. Every tile of a launch is run by exactly one workgroup, whatever the
 //      tile count, grid size and chunk size.
+//      The same for launches of one tile per workgroup, whose balanced chunk also leaves no
+//      XCD with more rounds than an even deal.
 //   2. The launcher's grid keeps every workgroup within the LDS row table,
 //      for any row table size, group sizes, M and CU count, at the kernel's
 //      real tile count (which the launcher bounds from above).
@@ -49,6 +51,32 @@ int main() {
       }
     }
   }
+  // 1b. one tile per workgroup, on the grid and balanced chunk of the medium-problem launcher
+  for (int cus : {8, 80, 256, 304}) {
+    for (int tiles = 1; tiles <= 20000; tiles += (tiles < 1200 ? 1 : 173)) {
+      const int chunk = sched_balanced_chunk(tiles, cus);
+      if (chunk < 1 || chunk > kTileChunk) return fail("chunk out of range", cus, tiles, chunk);
+      const long long even = ((tiles + kXcds - 1) / kXcds + cus / kXcds - 1) / (cus / kXcds);
+      // the kernel's tile count may be below the launcher's bound
+      for (int total : {tiles, tiles - tiles / 3, tiles / 2}) {
+        const long long nwg = sched_single_workgroups(tiles, chunk);
+        if (nwg % kXcds || nwg < tiles) return fail("one-tile grid", cus, tiles, nwg);
+        seen.assign(total, 0);
+        long long sum = 0;
+        for (long long i = 0; i < nwg; ++i) {
+          const int w = sched_tile_index((int)(i & 7), (int)(i >> 3), 0, 1, chunk);
+          if (w < 0) return fail("one-tile index out of range", cus, tiles, w);
+          if (w >= total) continue;
+          if (seen[w]++) return fail("one-tile launch runs a tile twice", cus, tiles, w);
+          ++sum;
+        }
+        if (sum != total) return fail("one-tile launch loses tiles", cus, tiles, sum);
+      }
+      for (int x = 0; x < kXcds; ++x)
+        if (sched_xcd_tiles(tiles, x, chunk) > even * (cus / kXcds))
+          return fail("uneven deal", cus, tiles, x);
+    }
+  }
   // 2. the launcher's grid respects the row table at the real tile count
   std::mt19937 rng(1234);
   const int BM = 256;
@@ -71,13 +99,26 @@ int main() {
         }
         const long long upper = ((long long)(M + BM - 1) / BM + G) * nt;
         if (total > upper) return fail("tile count above the launcher's bound", M, G, total);
-        const int chunk = sched_chunk((int)(rng() % 5), nt);  // 0: the default size
-        const long long nwg = sched_workgroups(upper, cus, rt, chunk);
+        const int chunk = sched_chunk((int)(rng() % 5), nt, (int)upper, cus);  // 0: balanced
+        const long long nwg = sched_persistent_workgroups(upper, cus, rt, chunk);
         if (nwg % kXcds || nwg < kXcds) return fail("grid not a multiple of 8", upper, cus, nwg);
         if (sched_max_tiles((int)total, (int)nwg, chunk) > rt)
           return fail("workgroup beyond the row table", total, nwg, rt);
         if (sched_max_tiles((int)upper, (int)nwg, chunk) > rt)
           return fail("bound beyond the row table", upper, nwg, rt);
+        // every tile exactly once on that grid and chunk
+        seen.assign(total, 0);
+        for (int i = 0; i < nwg; ++i) {
+          const int per = (int)nwg / kXcds, x = i & 7, slot = i >> 3;
+          const int n = sched_slot_tiles(sched_xcd_tiles((int)total, x, chunk), slot, per);
+          for (int t = 0; t < n; ++t) {
+            const int w = sched_tile_index(x, slot, t, per, chunk);
+            if (w < 0 || w >= total) return fail("persistent tile index", total, nwg, w);
+            if (seen[w]++) return fail("persistent launch runs a tile twice", total, nwg, w);
+          }
+        }
+        if (std::count(seen.begin(), seen.end(), 1) != total)
+          return fail("persistent launch loses tiles", total, nwg, chunk);
       }
     }
   }

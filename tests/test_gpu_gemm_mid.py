@@ -145,3 +145,29 @@ def test_row_major_overlapping_offsets(dsk):
     _check(out[5:90], x[5:90], w[0])
     _check(out[130:300], x[130:300], w[2])
     assert bool((out[:5] == 0).all() and (out[300:] == 0).all())
+
+
+@pytest.mark.parametrize("G,M", [(8, 1000), (16, 1000), (30, 1900)])
+def test_row_major_offsets_that_overlap_whole_groups(dsk, G, M):
+    """Offsets 0, M, 0, M, ...: every other group is all M rows, so the tiles are several times
+    the grid and a workgroup runs tile after tile, the staging of one against the DMA of the
+    next. All groups have the same weights, so each row has one right value."""
+    off = torch.tensor(([0, M] * G)[:G + 1], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(G)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.2).to(torch.bfloat16).to(DEV)  # noqa: E731
+    w1, w2 = rnd(384, 192).expand(G, 384, 192).contiguous(), rnd(256, 192).expand(G, 256, 192).contiguous()
+    x = rnd(M, 192)
+    rows = 64 if M // G <= 70 else 128
+    tiles = (G // 2) * -(-M // rows)
+    assert tiles > -(-M // rows) + G + 8      # more than the grid, rounded up to the XCDs
+    for _ in range(3):
+        gu = dsk.moe_gemm1(x, w1, off)
+        _check(gu, x, w1[0])
+        a = x.double() @ w1[0].double().t()
+        ref = torch.nn.functional.silu(a[:, :192]) * a[:, 192:]
+        h = dsk.moe_gemm1_swiglu(x, w1, off)
+        # rounding of h (2^-8), the hardware exp and reciprocal and K fp32 roundings: per element
+        room = a[:, :192].abs() * a[:, 192:].abs()
+        assert bool(((h.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * (room + 1)).all())
+        y = dsk.moe_gemm2(h, w2, off)
+        _check(y, h, w2[0])
