@@ -11,13 +11,17 @@
 // dot products.
 //
 // One workgroup per B tokens x B experts (B = 32, or 16 of the MFMA's 32 rows with
-// the others repeating them), 16 waves splitting K sixteen ways; each wave issues all
+// the others repeating the last, which a load merges; repeating all 16 cost up to half
+// as much again), 16 waves splitting K sixteen ways; each wave issues all
 // loads of a chunk of 8 K steps before its MFMAs. A workgroup pulls 2 B rows of x and
 // weights through one CU, which holds ~64 lines in flight, so that stream is its time:
-// blocks of 16 halve it and spread the work over four times the CUs (T = 32 and 600:
-// 16.1 us with blocks of 32, 11.1 and 11.6 with 16); from 2048 tokens up the blocks of 32
-// cover the CUs and read x half as often. The partial sums meet in LDS in a fixed order (waves 1..15 into
-// wave 0), so the result is the same on every run.
+// blocks of 16 halve it and spread the work over four times the CUs (64 experts,
+// H = 7168, T = 16 and 1024: 27.3 and 32.8 us with blocks of 32, 20.6 and 20.9 with 16;
+// at H = 2048 all of them are within the host's 10-12 us per call). They are taken while
+// a CU gets one block at most: with a second one in turn the blocks of 32 are ahead
+// (T = 1100 to 2047: 36-38 us, blocks of 16 60 us). The partial sums meet in LDS in a
+// fixed order (waves 1..15 into wave 0), so the result is the same on every run and for
+// either block.
 #include "dsk_internal.hpp"
 #include "gate_parts.hpp"
 #include "route_token.hpp"
@@ -37,7 +41,7 @@ __global__ __launch_bounds__(64 * kGateWaves) void gate_logits_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int t0 = blockIdx.x * B, e0 = blockIdx.y * B;
-  const int r32 = lane & (B - 1), h = lane >> 5;
+  const int r32 = min(lane & 31, B - 1), h = lane >> 5;
   // weights are MFMA operand A (output rows = experts), tokens operand B
   const int e = min(e0 + r32, E - 1);
   const int t = min(t0 + r32, T - 1);
@@ -128,7 +132,7 @@ int gate_parts_count(int T, int E, int H) {
 int launch_gate_logits(const uint16_t* x, int64_t ld_x, const uint16_t* wg, bool tiled,
                        const float* bias, float* logits, int64_t ld_out, int T, int E, int H,
                        hipStream_t st) {
-  const int B = T < 2048 ? 16 : 32;
+  const int B = (int64_t)((T + 15) / 16) * ((E + 15) / 16) <= num_cus() ? 16 : 32;
   dim3 grid((T + B - 1) / B, (E + B - 1) / B);
   auto kern = B == 16 ? (tiled ? gate_logits_kernel<true, 16> : gate_logits_kernel<false, 16>)
                       : (tiled ? gate_logits_kernel<true, 32> : gate_logits_kernel<false, 32>);
