@@ -240,9 +240,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
   };
 
   // DMA lane mapping: lane l lands at row l / CPR of its instruction's row group
-  // (RPI rows; group index islot + NI*i), physical chunk l % CPR
+  // (RPI rows; group index islot + NI*i), physical chunk l % CPR. The row is kept as a
+  // constant plus dma_r0, known to be below the step: the rows and columns of a wave's 8
+  // instructions then share their registers.
   const int islot = wave - (NW - NI);  // issuing slot 0 .. NI-1, negative if not issuing
   const int dma_row = lane / CPR;
+  constexpr int DMA_STEP = RPI * NI;
+  static_assert((DMA_STEP & (DMA_STEP - 1)) == 0, "a power of two");
+  const int dma_r0 = (RPI * islot + dma_row) & (DMA_STEP - 1);
   int dma_chunk;
   if constexpr (CPR == 8) dma_chunk = (lane & 7) ^ dma_row ^ (islot & 1);
   else dma_chunk = (lane & 3) ^ ((lane >> 4) & 3);
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
     if (!issuer) return;
 #pragma unroll
     for (int i = 0; i < A_INSTS; ++i) {
-      const int r = RPI * (islot + NI * i) + dma_row;
+      const int r = DMA_STEP * i + dma_r0;
       int row;
       if constexpr (GATHER) {
         row = s_rows[t_idx * BM + r];
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
         }
         b_off[i] = (uint32_t)((((int64_t)rb * (p.K / 16) + ksl) * 512 + lane * 8) * 2);
       } else {
-        const int r = RPI * (islot + NI * i) + dma_row;
+        const int r = DMA_STEP * i + dma_r0;
         int brow, col;
         if constexpr (SWIGLU) {
           const int wn = r / WN, w = r % WN;
@@ -367,7 +372,30 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
       for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.f;
 
   bf16x8_t fb[2][TN], fa[2][TM];
+  // Row-major weights: both operands are swizzled rows, and with an address per K step and
+  // operand kept over the loop the kernel spilled 30-50 registers, some reloaded in the loop
+  // of three row blocks, where a reload waits for the DMA just issued. The chunk of K step
+  // kk is at (the address of step 0) ^ 32 kk, so one register per operand is kept, hidden
+  // from the compiler's hoisting. No spills: grouped GEMM of 64 groups, K = 2048, N = 2816,
+  // 375 rows each 413 -> 335 us, 512 rows 391 -> 380.
+  const uint32_t frag_x = (uint32_t)lds_swz<CPR>(lane & 31, lane >> 5) * 16;
+  const uint32_t frag_a0 = lds_base + (uint32_t)(wave_m * WM) * BK * 2 + frag_x;
+  const uint32_t frag_b0 = lds_base + Cfg::A_BYTES + (uint32_t)(wave_n * WN) * BK * 2 + frag_x;
   auto read_frags = [&](int set, int stage, int kk) {
+    if constexpr (!TILED && CPR == 8) {
+      typedef const __attribute__((address_space(3))) bf16x8_t lds_frag_t;
+      uint32_t a = frag_a0, b = frag_b0;
+      asm volatile("" : "+v"(a), "+v"(b));
+      a = (a ^ (32 * kk)) + stage * Cfg::STAGE_BYTES;
+      b = (b ^ (32 * kk)) + stage * Cfg::STAGE_BYTES;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        fb[set][j] = *reinterpret_cast<lds_frag_t*>((uintptr_t)(b + 32 * j * BK * 2));
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        fa[set][i] = *reinterpret_cast<lds_frag_t*>((uintptr_t)(a + 32 * i * BK * 2));
+      return;
+    }
     const u32x4_t* As = lds4 + stage * (Cfg::STAGE_BYTES / 16);
     const u32x4_t* Bs = As + Cfg::A_BYTES / 16;
     const int ch = 2 * kk + (lane >> 5);
@@ -477,7 +505,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
               float v[4];
               // Read as plain values: at 2 waves per SIMD the 512 registers are one
               // file, and a read constrained to AGPRs (acc_read) had the compiler
-              // cut each wave's 256 into halves of 128, with 5 spills; now 241
+              // cut each wave's 256 into halves of 128, with 5 spills; now 234
               // and none. GEMM1 of 8192 tokens 656 -> 645 us, of 4096 362 -> 357.
 #pragma unroll
               for (int c = 0; c < 4; ++c) {
