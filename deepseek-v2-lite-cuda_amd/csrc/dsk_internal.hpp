@@ -24,6 +24,8 @@ struct GemmArgs {
                            // (0: unknown, M is used); selects the small-group kernel
   int offsets_sorted;      // offsets never decrease (the fused layer's own): the small-
                            // group grid then launches min(G, M) group ordinals, else G
+  int even_groups;         // every group is expected to hold about M / G rows (a layer with
+                           // no always-on groups, which hold all tokens); kernel choice only
   int chunk_m_tiles;       // large-group kernels: M tiles of a typical group, so that
                            // tiles are dealt to the XCDs a group at a time (0: chunks of
                            // up to kTileChunk tiles; gemm_sched.hpp)

@@ -395,6 +395,31 @@ static int launch_mid(const GemmArgs& a, hipStream_t st) {
   return check_launch("mid_gemm_kernel");
 }
 
+// Whether the 256 x 256 kernels are ahead for groups of about avg rows each (tiled weights,
+// no always-on groups among them). A group of just over 128 rows is two tiles here and one
+// there, and the time goes in rounds of a tile per CU, one here taking 1 / 1.9 of one there.
+// Measured on MI355X, us, here / there:
+//   64 experts of 1408, H = 2048, top-6: GEMM1  T = 1200 153 / 174, 1500 191 / 179, 1900
+//     201 / 188, 3000 257 / 289, 3500 270 / 295;  GEMM2  T = 1000 78 / 83, 1200 98 / 85,
+//     1500 101 / 92, 1900 108 / 99
+//   32 of 2048, H = 4096, top-2: GEMM1  T = 2100 263 / 241, 3000 272 / 263;  GEMM2  134 / 115,
+//     144 / 129
+//   16 of 4096, H = 2048, top-2: GEMM1  T = 1100 136 / 127, 2500 191 / 215, 3300 238 / 227
+//   8 of 1408, H = 2048, top-1:  GEMM1  T = 1500 32 / 42, 2500 44 / 41, 3000 53 / 45
+//   8 of 14336, H = 4096, top-2: GEMM1  T = 600 424 / 434, 1500 678 / 679, 1700 763 / 726
+// From 200 to 256 rows some groups pass 256 and both orders were seen (64 experts top-6,
+// T = 2300 205 / 194 and, with other logits, 205 / 233; top-1, T = 14000 211 / 245): left here.
+static bool even_groups_want_large(const GemmArgs& a, bool swiglu, int64_t avg) {
+  if (avg <= (swiglu ? 128 : 100) || (avg > 200 && avg <= 256)) return false;
+  const int64_t cus = num_cus(), nt = (a.N + (swiglu ? 127 : 255)) / (swiglu ? 128 : 256);
+  auto rounds = [&](int64_t rows, int64_t bm) {
+    return (a.G * nt * ((rows + bm - 1) / bm) + cus - 1) / cus;
+  };
+  // GEMM2's 512 tiles (64 groups, two on each CU) take a third one from the few groups past
+  // 128 rows that 100 rows on average bring
+  return 10 * rounds(avg + (swiglu ? 0 : 28), 128) > 19 * rounds(avg, 256);
+}
+
 bool mid_gemm_takes(const GemmArgs& a, bool swiglu) {
   const bool gather = a.a_rows != nullptr, grouped = a.offsets != nullptr;
   if (a.N % 32 || a.up_row_offset % 32 || !aligned16(a.C) || a.ldc % 8) return false;
@@ -415,7 +440,8 @@ bool mid_gemm_takes(const GemmArgs& a, bool swiglu) {
   if (!a.b_tiled) return avg <= 130;
   // tiled weights come from the fused layer, whose offsets never overlap (the grid holds
   // the tiles of such offsets only)
-  return swiglu == gather && a.offsets_sorted && avg <= (swiglu ? 430 : 230);
+  return swiglu == gather && a.offsets_sorted && avg <= (swiglu ? 430 : 230) &&
+         !(a.even_groups && even_groups_want_large(a, swiglu, avg));
 }
 
 int run_mid_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
@@ -435,8 +461,13 @@ int run_mid_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
   if (swiglu) return launch_mid<4, 2, true, true, true>(a, st);
   if (a.offsets != nullptr) {
     // few rows per group: 64-row tiles, and half the weight rows per workgroup, which
-    // spreads the weight stream over twice the workgroups (T = 250: 76 us against 91)
-    if (avg <= 80) return launch_mid<2, 1, false, false, true>(a, st);
+    // spreads the weight stream over twice the workgroups (T = 250: 76 us against 91). Even
+    // groups of more than 50 rows begin to pass 64, and stay whole where one 128-row tile
+    // each is at most two per CU but covers them (64 experts top-6, no always-on groups:
+    // T = 600 81 us with 64 rows, 73 with 128; 700 94, 74; 800 96, 75).
+    const int64_t wide = a.G * (int64_t)((a.N + 255) / 256), ncu = num_cus();
+    const bool whole = a.even_groups && avg > 50 && wide >= ncu && wide <= 2 * ncu;
+    if (avg <= 80 && !whole) return launch_mid<2, 1, false, false, true>(a, st);
     return launch_mid<4, 2, false, false, true>(a, st);
   }
   // Dense: the tile with the least estimated time, from c = tiles on the fullest CU.

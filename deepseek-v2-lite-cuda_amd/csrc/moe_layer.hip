@@ -140,6 +140,7 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
     g1.max_group_rows = T;  // a token routes to an expert at most once; shared groups hold T
     g1.b_tiled = weight_layout == DSK_LAYOUT_TILED;
     g1.chunk_m_tiles = chunk_m_tiles;
+    g1.even_groups = nsh == 0;
     if ((rc = run_gemm(g1, true, st))) return rc;
   }
   if ((rc = mark(2))) return rc;
@@ -160,6 +161,7 @@ static int layer_after_gate(const float* logits, int n_parts, int64_t part_strid
     g2.max_group_rows = T;
     g2.b_tiled = weight_layout == DSK_LAYOUT_TILED;
     g2.chunk_m_tiles = chunk_m_tiles;
+    g2.even_groups = nsh == 0;
     if ((rc = run_gemm(g2, false, st))) return rc;
     if ((rc = mark(3))) return rc;
 

@@ -78,7 +78,42 @@ def test_row_statistics(dsk, M):
 def test_fused_layer_groups(dsk, T, bias):
     """The grouped forms in the fused layer: equal and very unequal groups (some empty, some
     of nearly T rows) against per-expert products of the routing it returns."""
-    E, K, H, I, nsh = 16, 4, 256, 192, 2
+    _fused_layer_groups(dsk, T, bias, 16, 4, 256, 192, 2)
+
+
+@pytest.mark.parametrize("T,bias", [(500, 0.0), (700, 0.0), (700, 3.0), (1070, 0.0), (1300, 0.0),
+                                    (1500, 0.0), (1500, 4.0), (2130, 0.0), (2140, 0.0)])
+def test_fused_layer_groups_without_always_on(dsk, T, bias):
+    """64 experts and none always on, on both sides of the row counts where whole 128-row tiles
+    and the 256 x 256 kernels are taken (50, 80, 100, 128 and 200 rows per group)."""
+    _fused_layer_groups(dsk, T, bias, 64, 6, 1024, 512, 0)
+
+
+def test_time_of_groups_past_64_rows(dsk):
+    """A layer of 800 tokens on 64 routed experts (75 rows each) in less time than of 1000:
+    GEMM1 + GEMM2 222 and 229 us; 239 and 230 when the groups took two 64-row tiles."""
+    E, K, H, I = 64, 6, 2048, 1408
+    w1, w2 = (dsk.tile_weights((torch.randn(*s, device=DEV) * 0.02).to(torch.bfloat16))
+              for s in ((E, 2 * I, H), (E, H, I)))
+
+    def us(T):
+        x = torch.randn(T, H, device=DEV).to(torch.bfloat16)
+        logits = torch.randn(T, E, device=DEV)
+        best = float("inf")
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                dsk.moe_fused_forward_logits(logits, x, w1, w2, K, 0, E)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    us(1000)
+    assert us(800) < us(1000)
+
+
+def _fused_layer_groups(dsk, T, bias, E, K, H, I, nsh):
     g = torch.Generator().manual_seed(T)
     rnd = lambda *s, std=0.08: (torch.randn(*s, generator=g) * std).to(torch.bfloat16).to(DEV)  # noqa: E731
     x, wg = rnd(T, H, std=1.0), rnd(E, H)
