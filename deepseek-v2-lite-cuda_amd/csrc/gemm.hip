@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void grouped_gemm_kernel
 }
 
 // ------------------------------------------- large groups, tiled weights ----
-// Grouped GEMM for fragment-tiled weights, one wave per SIMD. A tile is 256
+// The layer's second GEMM on fragment-tiled weights, one wave per SIMD. A tile is 256
 // token rows x 256 weight rows; each of the 4 waves owns 64 weight rows (two
 // 32-row fragments) against all 256 token rows: 8 x 2 blocks of 32 x 32, 256
 // fp32 accumulators per lane in the accumulator registers.
@@ -582,19 +582,15 @@ constexpr int kWideBK = 64;                            // K per stage
 constexpr int kWideRing = 4;                           // token stages in the LDS ring
 constexpr int kWideStageBytes = kWideBM * kWideBK * 2;  // 32 KB
 constexpr int kWideRingBytes = kWideRing * kWideStageBytes;
-constexpr int kWideRowTiles = (kLdsPerCU - kWideRingBytes - 4096) / (kWideBM * 4);
-constexpr int kWideLdsBytes = kWideRingBytes + kWideRowTiles * kWideBM * 4;
 
-template <bool SWIGLU, bool GATHER>
 __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs p) {
   constexpr int TM = kWideBM / 32;     // token blocks per tile
   constexpr int TN = 2;                // weight blocks per wave
   constexpr int KSTEPS = kWideBK / 16;
-  constexpr int OUT_N = SWIGLU ? 32 * kWideWaves : 64 * kWideWaves;  // output columns per tile
+  constexpr int OUT_N = 64 * kWideWaves;  // output columns per tile
   constexpr int RPI = 8;               // token rows per 1 KB DMA instruction
   constexpr int A_INSTS = kWideBM / (kWideWaves * RPI);  // per wave per stage
   static_assert(A_INSTS == 2 * KSTEPS, "two DMA instructions per K step");
-  constexpr int THREADS = 64 * kWideWaves;
 
   extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
   __shared__ int s_inc[kMaxGroups];
@@ -604,18 +600,15 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int G = p.offsets != nullptr ? p.G : 1;
+  const int G = p.G;
   const int NT = (p.N + OUT_N - 1) / OUT_N;
 
   // ---- group table (as in grouped_gemm_kernel): row ranges, even M split
   if (tid < kMaxGroups) {
     int cnt = 0;
     if (tid < G) {
-      int mb = 0, me = p.M;
-      if (p.offsets != nullptr) {
-        mb = min(max(p.offsets[tid], 0), p.M);
-        me = min(max(p.offsets[tid + 1], mb), p.M);
-      }
+      const int mb = min(max(p.offsets[tid], 0), p.M);
+      const int me = min(max(p.offsets[tid + 1], mb), p.M);
       s_mb[tid] = mb;
       s_me[tid] = me;
       cnt = ((me - mb + kWideBM - 1) / kWideBM) * NT;
@@ -664,18 +657,6 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
   const int dma_chunk = (lane & 7) ^ dma_row ^ (wave & 1);  // row group wave + 4i: parity wave
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   const u32x4_t* lds4 = reinterpret_cast<const u32x4_t*>(lds);
-  const int row_limit = GATHER ? p.a_rows_limit : p.M;
-
-  int* s_rows = reinterpret_cast<int*>(lds + kWideRingBytes / 2);
-  if constexpr (GATHER) {
-    if (ntiles > kWideRowTiles) return;  // excluded by the launcher
-    for (int idx = tid; idx < ntiles * kWideBM; idx += THREADS) {
-      const Tile t = decode(idx / kWideBM);
-      const int m = t.m0 + idx % kWideBM;
-      s_rows[idx] = p.a_rows[m < t.me ? m : t.m0];
-    }
-    __syncthreads();
-  }
 
   // ---- token DMA cursor (three stages ahead of consumption)
   const char* Abase = reinterpret_cast<const char*>(p.A);
@@ -686,14 +667,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
 #pragma unroll
     for (int i = 0; i < A_INSTS; ++i) {
       const int r = RPI * (wave + kWideWaves * i) + dma_row;
-      int row;
-      if constexpr (GATHER) {
-        row = s_rows[t_idx * kWideBM + r];
-      } else {
-        const int m = t.m0 + r;
-        row = m < t.me ? m : t.m0;
-      }
-      row = (row >= 0 && row < row_limit) ? row : 0;
+      const int row = t.m0 + r < t.me ? t.m0 + r : t.m0;  // past the tile: its first row
       a_off[i] = (uint32_t)(((int64_t)row * p.lda + dma_chunk * 8) * 2);
     }
   };
@@ -726,13 +700,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
     const int last = p.N / 32 - 1;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      int rb;
-      if constexpr (SWIGLU) {
-        const int ob = min(t.n0 / 32 + wave, last);   // output block of this wave
-        rb = j == 0 ? ob : p.up_row_offset / 32 + ob;  // gate rows, then up rows
-      } else {
-        rb = min(t.n0 / 32 + TN * wave + j, last);
-      }
+      const int rb = min(t.n0 / 32 + TN * wave + j, last);
       b_off[j] = (uint32_t)((((int64_t)rb * (p.K / 16)) * 512 + lane * 8) * 2);
     }
   };
@@ -846,43 +814,36 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
     // each 32-row block and 4 consecutive columns per 4-register group, so
     // direct stores would touch 32 rows per instruction with 8 bytes each.
     // Instead each wave stages one block of its output (64 columns = 128 B
-    // per row; SwiGLU: 32 columns = 64 B) in its own 4 KB of the ring slot
-    // just consumed, and reads it back so that CHUNKS consecutive lanes hold
-    // one row segment: every store instruction writes whole row segments.
+    // per row) in its own 4 KB of the ring slot just consumed, and reads it
+    // back so that CHUNKS consecutive lanes hold one row segment: every store instruction writes whole row segments.
     // The slot is free until the next tile's DMA, which the barrier after
     // the epilogue holds back. The staging swizzle (16-byte chunk XOR row
     // bits, 8-byte half XOR row bit 4) keeps the 8-byte writes and the
     // 16-byte reads free of bank conflicts.
     {
-      constexpr int ROW_BYTES = SWIGLU ? 64 : 128;
+      constexpr int ROW_BYTES = 128;
       constexpr int CHUNKS = ROW_BYTES / 16;
       constexpr int ROWS_PER_INST = 64 / CHUNKS;
-      constexpr int JN = SWIGLU ? 1 : TN;
-      auto swz = [](int row) { return SWIGLU ? (row >> 2) & 3 : (row >> 1) & 7; };
+      auto swz = [](int row) { return (row >> 1) & 7; };
       char* stage_lds = reinterpret_cast<char*>(lds) + ((gc - 1) % kWideRing) * kWideStageBytes +
                         wave * 4096;
       const int r32 = lane & 31, h = lane >> 5;
-      const int col0 = SWIGLU ? ct.n0 + 32 * wave : ct.n0 + 64 * wave;  // this wave's columns
+      const int col0 = ct.n0 + 64 * wave;  // this wave's columns
       const int rl = lane / CHUNKS, cl = lane % CHUNKS;
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         if (i >= tma) continue;
 #pragma unroll
-        for (int j = 0; j < JN; ++j) {
+        for (int j = 0; j < TN; ++j) {
 #pragma unroll
           for (int qg = 0; qg < 4; ++qg) {
             float v[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              if constexpr (SWIGLU)
-                v[c] = silu_f(acc_read(acc[0][i][4 * qg + c])) * acc_read(acc[1][i][4 * qg + c]);
-              else
-                v[c] = acc_read(acc[j][i][4 * qg + c]);
-            }
+            for (int c = 0; c < 4; ++c) v[c] = acc_read(acc[j][i][4 * qg + c]);
             u32x2_t o;
             o[0] = pack_bf16x2(v[0], v[1]);
             o[1] = pack_bf16x2(v[2], v[3]);
-            const int chunk = SWIGLU ? qg : 4 * j + qg;
+            const int chunk = 4 * j + qg;
             const int off = r32 * ROW_BYTES + ((chunk ^ swz(r32)) * 16) + ((h ^ ((r32 >> 4) & 1)) * 8);
             *reinterpret_cast<u32x2_t*>(stage_lds + off) = o;
           }
@@ -1317,20 +1278,14 @@ static int launch_grouped_gemm(GemmArgs a, hipStream_t st) {
   return check_launch("grouped_gemm_kernel");
 }
 
-template <bool SWIGLU, bool GATHER>
 static int launch_wide_gemm(GemmArgs a, hipStream_t st) {
-  auto kern = wide_gemm_kernel<SWIGLU, GATHER>;
+  auto kern = wide_gemm_kernel;
   static std::once_flag once[kMaxDevices];
-  allow_lds(once, reinterpret_cast<const void*>(kern), kWideLdsBytes);
-  constexpr int OUT_N = SWIGLU ? 32 * kWideWaves : 64 * kWideWaves;
-  const int G = a.offsets != nullptr ? a.G : 1;
-  const int64_t nt = (a.N + OUT_N - 1) / OUT_N;
-  const int64_t upper = ((int64_t)(a.M + kWideBM - 1) / kWideBM + (a.offsets ? G : 0)) * nt;
-  const int64_t nwg = persistent_grid(a, upper, nt, GATHER ? kWideRowTiles : 0);
-  if (GATHER &&
-      (upper > INT32_MAX || sched_max_tiles((int)upper, (int)nwg, a.chunk) > kWideRowTiles))
-    return fail(DSK_ERR_INVALID_ARG, "wide_gemm: a workgroup's tiles exceed the LDS row table");
-  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(64 * kWideWaves), kWideLdsBytes, st, a);
+  allow_lds(once, reinterpret_cast<const void*>(kern), kWideRingBytes);
+  const int64_t nt = (a.N + 64 * kWideWaves - 1) / (64 * kWideWaves);
+  const int64_t upper = ((int64_t)(a.M + kWideBM - 1) / kWideBM + a.G) * nt;
+  const int64_t nwg = persistent_grid(a, upper, nt, 0);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(64 * kWideWaves), kWideRingBytes, st, a);
   return check_launch("wide_gemm_kernel");
 }
 
@@ -1425,14 +1380,15 @@ static int run_gemm_t(const GemmArgs& a, hipStream_t st) {
 #ifndef DSK_GEMM_WIDE
 #define DSK_GEMM_WIDE 1
 #endif
-  // fragment-tiled weights with K % 128 == 0 and 16-byte aligned output rows:
-  // one wave per SIMD, weights straight to registers. Measured on MI355X at
+  // groups on fragment-tiled weights with K % 128 == 0 and 16-byte aligned output
+  // rows: one wave per SIMD, weights straight to registers. Measured on MI355X at
   // T=4096: 234 us against 251 us for the down projection, but 448 against
   // 418 us for the gathered SwiGLU projection (368 against 360 us in steady
   // state), which stays on the 8-wave kernel.
-  if (DSK_GEMM_WIDE && TILED && !(SWIGLU && GATHER) && a.K % (2 * kWideBK) == 0 &&
-      aligned16(a.C) && a.ldc % 8 == 0)
-    return launch_wide_gemm<SWIGLU, GATHER>(a, st);
+  if constexpr (DSK_GEMM_WIDE && TILED && !SWIGLU && !GATHER) {
+    if (a.offsets != nullptr && a.K % (2 * kWideBK) == 0 && aligned16(a.C) && a.ldc % 8 == 0)
+      return launch_wide_gemm(a, st);
+  }
   constexpr int BM = DSK_GEMM_BM, BN = DSK_GEMM_BN, WM = DSK_GEMM_WAVES_M;
   constexpr int BK = DSK_GEMM_BK, ST = DSK_GEMM_STAGES;
   constexpr int WN = DSK_GEMM_WAVES_N;
@@ -1461,13 +1417,15 @@ int run_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
                 "linear_rowscale: need 1 or 2 parts, cols > 0 and ld_rowscale >= M");
     return run_mid_gemm(a, false, st);
   }
-  const bool g = a.a_rows != nullptr;
-  if (a.b_tiled) {
-    if (swiglu) return g ? run_gemm_t<true, true, true>(a, st) : run_gemm_t<true, false, true>(a, st);
-    return g ? run_gemm_t<false, true, true>(a, st) : run_gemm_t<false, false, true>(a, st);
-  }
-  if (swiglu) return g ? run_gemm_t<true, true, false>(a, st) : run_gemm_t<true, false, false>(a, st);
-  return g ? run_gemm_t<false, true, false>(a, st) : run_gemm_t<false, false, false>(a, st);
+  // the forms there are: SwiGLU on gathered rows (the fused layer), on rows in place (the op,
+  // row-major weights), and plain products on rows in place
+  const bool gather = a.a_rows != nullptr;
+  if (gather != swiglu && (gather || a.b_tiled))
+    return fail(DSK_ERR_INVALID_ARG, "grouped GEMM: no kernel for this form");
+  if (a.b_tiled)
+    return swiglu ? run_gemm_t<true, true, true>(a, st) : run_gemm_t<false, false, true>(a, st);
+  if (!swiglu) return run_gemm_t<false, false, false>(a, st);
+  return gather ? run_gemm_t<true, true, false>(a, st) : run_gemm_t<true, false, false>(a, st);
 }
 
 // A grouped GEMM op on a caller's offsets: rows that no group covers come out zero, in
