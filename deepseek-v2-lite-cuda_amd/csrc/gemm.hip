@@ -898,7 +898,13 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void wide_gemm_kernel(GemmArgs 
 // kernel, so the output layout per lane is the same (4 consecutive columns).
 constexpr int kSkinnyWaves = 4;  // waves per workgroup, each one slice of K
 constexpr int kSkinnyThreads = 64 * kSkinnyWaves;
-constexpr int kSkinnyMaxRows = 64;  // largest group the small-group kernel is chosen for
+// Largest group the small-group kernel is chosen for. Against the medium-problem kernel at
+// 33 to 64 tokens, layer of 64 + 2 experts top-6, GEMM1 + GEMM2, us: tiled weights, uniform
+// routing 33 tokens 116 + 62 / 131 + 67, 64 126 + 69 / 132 + 75, skewed routing (Zipf) 48
+// 45 + 23 / 41 + 22, 61 51 + 32 / 47 + 32; row-major weights 33 255 + 133 / 152 + 66, 64
+// 280 + 150 / 156 + 76, where the medium-problem kernel would be the better one from 33.
+// Tiled projections of 33 to 64 rows, through the op: N = 3648 11.8-12.9 / 13.4-13.6.
+constexpr int kSkinnyMaxRows = 64;
 // K steps (of 16) per load batch: 4 for one 32-row token block; 2 for two,
 // whose token fragments double the registers per step (measured on MI355X at
 // T=64: 117 us against 125 us per layer step with 4)
@@ -1310,12 +1316,13 @@ static int launch_skinny_gemm(const GemmArgs& a, hipStream_t st) {
     }
   }
   if constexpr (SWIGLU) {
-    // Fewer than two 32-column workgroups per CU (a call with 8 rows: 8 groups x
-    // 44): a CU's fetch rate bounds each workgroup's weight stream, so the CUs
-    // that hold two set the launch time. 16-column units halve the bytes per
-    // workgroup and spread them over the CUs more evenly. Measured on MI355X:
-    // GEMM1 at T = 1 27.7 -> 25.2 us (bitwise the same output); at T = 2-4 (704
-    // or more workgroups) unchanged, at T = 16 1.4 us and at T = 64 11 us slower.
+    // Fewer than two 32-column workgroups per CU (narrow experts, or few of them): a CU's
+    // fetch rate bounds each workgroup's weight stream, so the CUs that hold two set the
+    // launch time. 16-column units halve the bytes per workgroup and spread them over the
+    // CUs more evenly. Measured on MI355X, GEMM1 in 32- and 16-column units: 8 experts top-2,
+    // H = 4096, I = 1408 (352 workgroups) T = 4 35.4 / 30.9 us, 32 39.6 / 35.8, 64 42.0 /
+    // 42.1; 64 + 2 of 512, H = 2048, T = 3 21.8 / 19.0; 8 + 1 of 1408, H = 2048 (396) T = 4
+    // 21.3 / 18.3, 32 26.5 / 26.8, 64 32.4 / 37.0.
     if (GL * ((a.N + 31) / 32) < 2 * (int64_t)num_cus()) {
       const int n_blocks = (a.N + 15) / 16;
       hipLaunchKernelGGL((skinny_gemm_kernel<MT, true, GATHER, TILED, 1, kSkinnyWaves>),

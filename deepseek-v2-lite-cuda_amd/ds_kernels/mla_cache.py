@@ -203,7 +203,13 @@ class AbsorbedMLAWeights:
 
 # A step of at least this many new tokens (a prompt) attends through up-projected
 # K and V, like DeepSeekMLA.forward: the absorbed kernel reads every cached row
-# once per new token, which a long step cannot amortise.
+# once per new token, which a long step cannot amortise. Measured on MI355X, us per
+# step, up-projected / absorbed: one sequence, nothing cached, 64 tokens 114 / 54 (one
+# C call up to 64), 100 125 / 142, 128 125 / 139; 4000 cached 64 165 / 88, 128 179 /
+# 143, 200 179 / 206. 16 sequences, nothing cached, 5 tokens each 132 / 144, 100 131 /
+# 164, 128 131 / 178; 4000 cached 32 492 / 300, 64 515 / 541, 128 555 / 1038. The two
+# meet between 5 and 150 tokens depending on both; the line is one that long contexts
+# agree with, not the best for each.
 UP_PROJECTED_MIN_TOKENS = 128
 
 # Largest decode step (new tokens of all sequences) that runs as one C call.
