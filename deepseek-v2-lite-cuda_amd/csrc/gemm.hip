@@ -10,10 +10,10 @@
 // device-side offsets array (expert_offsets), so the host never waits for them.
 //
 // Scheduling: a persistent grid (one workgroup per CU). Output tiles are
-// enumerated group-major, then N-tile, then M-tile, and the enumeration is cut
-// into 8 contiguous ranges, one per XCD (workgroup i runs on XCD i % 8): the
-// M-tiles that share a weight tile run at about the same time on the same XCD,
-// so the weight tile is mostly re-read from that XCD's L2.
+// enumerated group-major, then N-tile, then M-tile, and dealt to the 8 XCDs in
+// chunks (gemm_sched.hpp; workgroup i runs on XCD i % 8): the M-tiles that share
+// a weight tile run at about the same time on the same XCD, so the weight tile
+// is mostly re-read from that XCD's L2.
 //
 // Data movement: each workgroup runs one continuous stream of K stages over
 // all of its tiles. A stage (BM token rows + BN weight rows, BK deep) lands in

@@ -1,11 +1,14 @@
 // Fused DeepSeekMoE forward on one GPU: the whole layer (moe.py:77-109) as one
-// C call that enqueues 4-6 kernels on the caller's stream and never waits.
+// C call that enqueues 2-6 kernels on the caller's stream and never waits.
 //
 //   [partial gate sums, dsk_moe_layer_forward only]  ->
 //   route (+histogram, ranks)  ->  [scan + permute, one kernel, when T > 64]  ->
 //   grouped GEMM1 + SwiGLU (A rows gathered from x through token_map)  ->
 //   grouped GEMM2  ->  combine (ascending-expert fp32 sum + shared rows, one
 //   bf16 rounding)
+//
+// One token routes inside its first GEMM; GEMM2 and the combine of one and two
+// tokens are one kernel (gemv.hip).
 //
 // The shared expert (intermediate 2*I) is run as n_shared_groups extra groups
 // of width I appended after the routed experts: group E+j holds gate/up rows
@@ -57,7 +60,7 @@ static FusedLayout fused_layout(int T, int E, int K, int nsh, int H, int I) {
 #endif
 // M tiles (of 256 rows) of a typical routed group, for dealing the large-group
 // GEMMs' tiles to the XCDs one routed group at a time (GemmArgs::chunk_m_tiles),
-// or 0 (chunks of the default size) where that deal would not be even: the E
+// or 0 (the balanced deal's chunks) where that deal would not be even: the E
 // routed groups make E chunks and the always-on groups (T rows each) must fill
 // whole chunks, the count of all chunks a multiple of the 8 XCDs. At T = 4096
 // (E = 64, K = 6, 2 always-on groups): 2 M tiles, 64 + 16 chunks.

@@ -264,8 +264,10 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
 // earlier tokens in the LDS (integer sums, so every workgroup agrees), which with the
 // given offsets and the order inside the workgroup makes its slots, and copies its rows,
 // each read once for its K slots. Replaces four launches (rank, scan, permute, gather),
-// whose latency, not their work, was the time: T = 600 18.6 -> 11.3 us; at T = 4096 the
-// counting costs about what the launches did.
+// whose latency, not their work, was the time. Through the op, top-6 of 64, us: T = 600
+// 25.4 -> 17.1, 2500 25.4 -> 18.9, 4096, at the line, 32.9 -> 24.9 (rows of 14 KB 113.7 ->
+// 106.5, one expert each 25.3 -> 17.2); larger counts were not measured, and every earlier
+// token is counted again by every workgroup.
 constexpr int kDispatchTokens = 4;
 constexpr int kDispatchMaxTokens = 4096;
 
