@@ -71,3 +71,20 @@ def assert_routing_admissible(idx: np.ndarray, lg64: np.ndarray, bound: np.ndarr
     b = 2 * bound.max(axis=1, keepdims=True)
     assert np.all(np.abs(chosen - s) <= b), "routing choice outside the fp32 error bound"
     assert all(len(set(r)) == len(r) for r in idx.tolist()), "an expert chosen twice"
+
+
+def best_times(*fns, calls=20, rounds=10):
+    """Shortest time of `calls` calls of each function, in ms, the functions in turn (so that
+    clock changes meet all of them), after one round of each."""
+    best = [float("inf")] * len(fns)
+    for r in range(rounds + 1):
+        for i, fn in enumerate(fns):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(calls):
+                fn()
+            b.record()
+            b.synchronize()
+            if r:
+                best[i] = min(best[i], a.elapsed_time(b))
+    return best

@@ -12,7 +12,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from gpu_util import BF16_TOL, F32_TOL, max_rel_err, np32
+from gpu_util import BF16_TOL, F32_TOL, best_times, max_rel_err, np32
 from oracle import moe as om
 
 pytestmark = pytest.mark.gpu
@@ -78,22 +78,11 @@ def test_gate_logits_blocks(dsk, E):
 def test_gate_logits_time_past_one_block_per_cu(dsk):
     """1500 tokens in less time than 2048 and a quarter (H = 7168: 38 and 36 us; 60 us when
     blocks of 16 went on past one for each CU)."""
-    x = torch.randn(2048, 7168, device=DEV, dtype=torch.bfloat16)
-    wg = torch.randn(64, 7168, device=DEV, dtype=torch.bfloat16)
-
-    def us(T):
-        best = float("inf")
-        for _ in range(8):
-            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            a.record()
-            for _ in range(20):
-                dsk.moe_gate(x[:T], wg)
-            b.record()
-            b.synchronize()
-            best = min(best, a.elapsed_time(b))
-        return best
-    us(2048)
-    assert us(1500) < 1.25 * us(2048)
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(2048, 7168, generator=g).to(torch.bfloat16).to(DEV)
+    wg = torch.randn(64, 7168, generator=g).to(torch.bfloat16).to(DEV)
+    few, many = best_times(lambda: dsk.moe_gate(x[:1500], wg), lambda: dsk.moe_gate(x, wg))
+    assert few < 1.25 * many, (few, many)
 
 
 # ------------------------------------------------------------------ routing --
@@ -258,18 +247,12 @@ def test_combine_many_slots_per_token_time(dsk):
     """128 slots per token, 268 MB of rows: 0.16 ms, and 8.1 ms when the tokens past a
     workgroup's list searched the map one slot at a time."""
     T, S, H = 512, 65536, 2048
+    g = torch.Generator().manual_seed(0)
     y = torch.randn(S, H, device=DEV, dtype=torch.bfloat16)
-    tm = torch.randint(0, T, (S,), device=DEV, dtype=torch.int32)
-    dw = torch.rand(S, device=DEV)
-    best = float("inf")
-    for _ in range(5):
-        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        a.record()
-        dsk.moe_combine(y, tm, dw, T)
-        b.record()
-        b.synchronize()
-        best = min(best, a.elapsed_time(b))
-    assert best < 1.5, f"{best:.2f} ms"
+    tm = torch.randint(0, T, (S,), generator=g, dtype=torch.int32).to(DEV)
+    dw = torch.rand(S, generator=g).to(DEV)
+    ms, = best_times(lambda: dsk.moe_combine(y, tm, dw, T), calls=2, rounds=5)
+    assert ms / 2 < 1.5, ms / 2
 
 
 @pytest.mark.parametrize("T", [1, 3, 4, 5, 257, 4096, 4097])
