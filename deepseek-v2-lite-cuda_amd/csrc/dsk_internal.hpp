@@ -11,6 +11,8 @@ struct GemmArgs {
   int64_t lda;
   const int32_t* a_rows;   // optional: A row of output row m is a_rows[m]
   int a_rows_limit;        // valid A rows are [0, a_rows_limit)
+  int even_groups;         // every group is expected to hold about M / G rows (a layer with
+                           // no always-on groups, which hold all tokens); kernel choice only
   const uint16_t* B;
   int64_t ldb;
   int64_t b_group_stride;  // elements between consecutive groups' weights
@@ -24,8 +26,6 @@ struct GemmArgs {
                            // (0: unknown, M is used); selects the small-group kernel
   int offsets_sorted;      // offsets never decrease (the fused layer's own): the small-
                            // group grid then launches min(G, M) group ordinals, else G
-  int even_groups;         // every group is expected to hold about M / G rows (a layer with
-                           // no always-on groups, which hold all tokens); kernel choice only
   int chunk_m_tiles;       // large-group kernels: M tiles of a typical group, so that
                            // tiles are dealt to the XCDs a group at a time (0: chunks of
                            // up to kTileChunk tiles; gemm_sched.hpp)

@@ -74,9 +74,11 @@ __device__ __forceinline__ void mid_tile(const GemmArgs& p, int W, int NT, char*
   const int nblk = (gme - mb + 31) / 32;
   int nt, mi;
   sched_group_tile(local, mt, NT, &nt, &mi);
+  // the even split of the blocks; the product fits 32 bits up to kMidMaxRows (sched_tile_block
+  // holds for any count, at 0.1-0.2 us a launch)
   nt = __builtin_amdgcn_readfirstlane(nt);
-  const int m0 = __builtin_amdgcn_readfirstlane(mb + 32 * sched_tile_block(mi, mt, nblk, TM));
-  const int me = __builtin_amdgcn_readfirstlane(min(mb + 32 * sched_tile_block(mi + 1, mt, nblk, TM), gme));
+  const int m0 = __builtin_amdgcn_readfirstlane(mb + 32 * (mi * nblk / mt));
+  const int me = __builtin_amdgcn_readfirstlane(min(mb + 32 * ((mi + 1) * nblk / mt), gme));
   const int n0 = nt * OUT_N;
   const int tma = (me - m0 + 31) / 32;  // token blocks with rows
   const int nk = p.K / kMidBK;
@@ -382,6 +384,7 @@ __global__ __launch_bounds__(kMidThreads, 2) void mid_gemm_kernel(GemmArgs p, in
 
 template <int TM, int TN, bool SWIGLU, bool GATHER, bool TILED>
 static int launch_mid(const GemmArgs& a, hipStream_t st) {
+  if (a.M > kMidMaxRows) return fail(DSK_ERR_INVALID_ARG, "mid_gemm: too many rows");
   constexpr int OUT_N = MidCfg<TM, TN, SWIGLU, GATHER, TILED>::OUT_N;
   const int64_t nt = (a.N + OUT_N - 1) / OUT_N;
   const int64_t tiles =
@@ -437,6 +440,7 @@ bool mid_gemm_takes(const GemmArgs& a, bool swiglu) {
   //   gate|up  T = 16 124 / 181, 150 156 / 209, 600 164 / 219, 1000 191 / 222, 2000 260 / 239
   //   down     T = 16 50 / 91, 150 67 / 101, 600 80 / 106, 1000 86 / 108, 2000 127 / 119
   const int64_t avg = a.M / (a.G > 0 ? a.G : 1);
+  if (a.M > kMidMaxRows) return false;
   if (!a.b_tiled) return avg <= 130;
   // tiled weights come from the fused layer, whose offsets never overlap (the grid holds
   // the tiles of such offsets only)
@@ -445,6 +449,19 @@ bool mid_gemm_takes(const GemmArgs& a, bool swiglu) {
 }
 
 int run_mid_gemm(const GemmArgs& a, bool swiglu, hipStream_t st) {
+  if (a.offsets == nullptr && a.M > kMidMaxRows) {  // a launch for each kMidMaxRows rows
+    for (int r = 0; r < a.M; r += kMidMaxRows) {
+      GemmArgs part = a;
+      part.M = a.M - r < kMidMaxRows ? a.M - r : kMidMaxRows;
+      part.A += (int64_t)r * a.lda;
+      part.C += (int64_t)r * a.ldc;
+      if (a.rowsq_out != nullptr) part.rowsq_out += r;
+      if (a.rowscale_ss != nullptr) part.rowscale_ss += r;
+      const int rc = run_mid_gemm(part, swiglu, st);
+      if (rc) return rc;
+    }
+    return DSK_OK;
+  }
   const int64_t avg = a.M / (a.offsets != nullptr && a.G > 0 ? a.G : 1);
   const bool gather = a.a_rows != nullptr;
   if (a.offsets != nullptr && !a.b_tiled) {

@@ -91,6 +91,10 @@ DSK_HD void sched_group_tile(int local, int mt, int nt_count, int* nt, int* mi) 
   *mi = p * kPanelM + (r - *nt * ps);
 }
 
+// Most rows of a launch of the medium-problem kernel, whose tiles take the split below as it
+// stands: at 64 rows a tile the product is at most 2^29.
+constexpr int kMidMaxRows = 1 << 20;
+
 // First 32-row block of M tile mi when a group's nblk blocks are split evenly over its
 // mt = ceil(nblk / tm) tiles of at most tm blocks: floor(mi * nblk / mt). That product
 // passes 2^31 from 2.1 million rows in tiles of two blocks, so it is taken apart:

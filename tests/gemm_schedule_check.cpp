@@ -148,6 +148,8 @@ int main() {
         }
       }
       if (sched_tile_block(mt, mt, nblk, tm) != nblk) return fail("row split end", rows, tm, mt);
+      if (rows <= kMidMaxRows && (long long)mt * nblk > INT32_MAX)
+        return fail("split of the medium-problem kernel", rows, tm, mt);
     }
   }
   std::printf("OK\n");

@@ -47,8 +47,9 @@ def test_dense(dsk, M, N, K):
     assert bool((guard[0] == 7).all() and (guard[M + 1] == 7).all() and (guard[:, N:] == 7).all())
 
 
-# rows times blocks past 2^31: 64-row tiles from 2.1 million rows, 128-row ones from 3.0
-@pytest.mark.parametrize("M,N", [(2200003, 128), (3100003, 256)])
+# several launches of 2^20 rows; in one, rows times blocks would pass 2^31 from 2.1 million
+# rows in 64-row tiles (N = 128), from 3.0 in 128-row ones
+@pytest.mark.parametrize("M,N", [((1 << 20) + 1, 128), (2200003, 128), (3100003, 256)])
 def test_dense_millions_of_rows(dsk, M, N):
     g = torch.Generator(device=DEV).manual_seed(N)
     x = torch.randn(M, 64, generator=g, device=DEV, dtype=torch.bfloat16)
@@ -73,6 +74,23 @@ def test_row_statistics(dsk, M):
     z = dsk.linear_rowscale(x, wt, ss, 512, 1e-6)
     r = torch.rsqrt(ss.double().sum(0) / 512 + 1e-6)[:, None]
     _check(z, x, w, r * (1 + 2.0 ** -20))
+
+
+def test_row_statistics_of_millions_of_rows(dsk):
+    """The sums of squares and the row scales of every launch's rows."""
+    M = (1 << 20) + 77
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(M, 128, generator=g, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(256, 128, generator=g, device=DEV).mul_(0.05).to(torch.bfloat16)
+    wt = dsk.tile_weights(w[None])[0]
+    y, ss = dsk.linear_rowsq(x, wt, 0, 256)
+    z = dsk.linear_rowscale(x, wt, ss, 256, 1e-6)
+    for r in (slice(0, 5000), slice(M - 5000, M)):
+        _check(y[r], x[r], w)
+        ref = y[r].double().square().sum(-1)
+        assert bool(((ss[0, r].double() - ref).abs() <= 256 * 2.0 ** -23 * ref).all())
+        s = torch.rsqrt(ss[0, r].double() / 256 + 1e-6)[:, None]
+        _check(z[r], x[r], w, s * (1 + 2.0 ** -20))
 
 
 @pytest.mark.parametrize("T,bias", [(65, 0.0), (150, 3.0), (600, 0.0), (600, 6.0), (1400, 3.0),
